@@ -108,7 +108,8 @@ int gen_copies(uint16_t* out, const ng_i64* copies, ng_i64 m, const uint16_t* sr
  * ------------------------------------------------------------------------------------------------------------ */
 
 /* one level's scan counted in a split table (keys EMPTY-filled, cnts zeroed); sparse 0: a lane per position, 1: a
- * lane per bitmap word, 2: the set positions listed per wave in LDS (bm_in required for 1 and 2); flags[0] = full */
+ * lane per bitmap word, 2: the set positions listed per wave in LDS, 4: as 0 or 2 by each wave's own positions' density
+ * (bm_in required for 1, 2 and 4); flags[0] = full */
 int ng_scan_count(const uint16_t* tok, ng_i64 L, int k, const uint32_t* bm_in, uint32_t* bm_out, const ng_u64* vt,
                   ng_u64 vcap, const uint32_t* vrep, const uint16_t* x, ng_u64* keys, uint32_t* cnts, ng_u64 cap,
                   uint32_t* flags, int grid, int sparse, void* stream);

@@ -352,6 +352,136 @@ __global__ void __launch_bounds__(256) scan_compact_k(const u16* __restrict__ to
     sink_end(sink, &ss);
 }
 
+// Gated levels whose density the host does not know (a build that has read no hit statistics: its first one, and every
+// one that never asks for them): the wave decides. A wave owns `per` consecutive groups of 64 gate words (2048
+// positions; ceil(L / (grid * 8192)) of them, so a block's hits fit ng_emit_region) and takes up to GATED_SPAN groups at
+// a time, their words loaded together. Where at least half of the span's positions are set it probes every position of
+// it as scan_dense_k does (a lane per position, no list to make); elsewhere it lists the set positions in LDS across the
+// span's groups and probes 256 at a time as soon as that many are listed, so that a sparse span costs one round of
+// probes and not one per group. Bound by the probes' random lines where the gate is dense, by the bitmaps (an eighth
+// of a byte read and written per position) where it is sparse. One copy of the probe code serves both (two took 130
+// registers, three waves a SIMD, and 15.3 ms at n = 3 against 12.9 with one at five waves; the longer keys of k > 4 spill
+// there, so they keep four). Measured (1e9 positions, no statistics): the scans of n = 3..8 took 56.2 ms behind
+// scan_dense_k alone, 21.1 ms here; where the densities are known, the host's choice of kernel takes 20.6 ms.
+#define GATED_SPAN 8
+#define GATED_PPL 4
+template <int K, class S>
+__global__ void __launch_bounds__(256, K >= 1 && K <= 4 ? 5 : 4) scan_gated_k(const u16* __restrict__ tok, i64 L, int k,
+                                                    const u32* __restrict__ bm_in, u32* __restrict__ bm_out,
+                                                    const u64* __restrict__ vt, u64 vcap, const u32* __restrict__ vrep,
+                                                    const u16* __restrict__ x, S sink, u32* flags, const u32* pre_flag) {
+    __shared__ u16 list[4][2048 + WAVE * GATED_PPL];
+    __shared__ u32 words[4][GATED_SPAN * WAVE];
+    __shared__ SinkShared ss;
+    sink_begin<S>(sink, &ss);
+    const int lane = lane_id(), w = threadIdx.x / WAVE;
+    const bool pre = pre_on(pre_flag);
+    const i64 nwords = (L + 31) >> 5;
+    const i64 ngroups = (nwords + WAVE - 1) / WAVE;
+    const i64 per = (ngroups + (i64)gridDim.x * 4 - 1) / ((i64)gridDim.x * 4);
+    const i64 gbeg = ((i64)blockIdx.x * 4 + w) * per;
+    const i64 gend = gbeg + per < ngroups ? gbeg + per : ngroups;
+    for (i64 g0 = gbeg; g0 < gend; g0 += GATED_SPAN) {
+        const int ng = gend - g0 < GATED_SPAN ? (int)(gend - g0) : GATED_SPAN;
+        const bool full = sink_full<S>(flags);
+        u32 raw[GATED_SPAN];
+#pragma unroll
+        for (int q = 0; q < GATED_SPAN; ++q) {
+            const i64 wi = (g0 + q) * WAVE + lane;
+            raw[q] = q < ng && wi < nwords ? bm_in[wi] : 0u;
+        }
+        u32 before = 0xFFFFFFFFu;  // the word before the span (the range's first word: its bit counts as set)
+        if (g0 > 0 && lane == 0) before = bm_in[g0 * WAVE - 1];
+        u32 total = 0;
+#pragma unroll
+        for (int q = 0; q < GATED_SPAN; ++q) {
+            u32 word = raw[q];
+            if (pre) {
+                u32 left = (u32)__shfl_up((int)raw[q], 1, WAVE);
+                if (lane == 0) left = before;
+                word &= (word << 1) | (left >> 31);
+                before = (u32)__shfl((int)raw[q], WAVE - 1, WAVE);
+            }
+            if (q < ng) words[w][q * WAVE + lane] = word;
+            total += (u32)__popc(word);
+        }
+#pragma unroll
+        for (int d = WAVE / 2; d > 0; d >>= 1) total += (u32)__shfl_xor((int)total, d, WAVE);
+        // the list and the words are the wave's own: no block barrier (the wave's LDS accesses stay in order)
+        const i64 p00 = (g0 * WAVE) << 5;
+        const bool dense = total >= (u32)ng * (WAVE * 16);
+        u32 n = 0;  // positions of the group (dense), or listed, that are not probed yet
+        for (int q = 0; total && q < ng; ++q) {
+            if (dense) {
+                n = WAVE * 32;
+            } else {
+                u32 bits = words[w][q * WAVE + lane];
+                words[w][q * WAVE + lane] = 0u;
+                u32 incl = (u32)__popc(bits);
+                u32 at = n - incl;
+#pragma unroll
+                for (int d = 1; d < WAVE; d <<= 1) {
+                    const u32 o = (u32)__shfl_up((int)incl, d, WAVE);
+                    if (lane >= d) incl += o;
+                }
+                at += incl;
+                n += (u32)__shfl((int)incl, WAVE - 1, WAVE);
+                while (bits) {
+                    const int b = __ffs(bits) - 1;
+                    bits &= bits - 1;
+                    list[w][at++] = (u16)((q * WAVE + lane) * 32 + b);
+                }
+            }
+            // the last 256 of them probed while there are that many (at the span's end: whatever is left), so at most
+            // 255 stay listed beside the next group's 2048
+            while (n >= WAVE * GATED_PPL || (n && q == ng - 1)) {
+                const u32 m = n < WAVE * GATED_PPL ? n : WAVE * GATED_PPL;
+                n -= m;
+                Walk2 wk[GATED_PPL];
+                u32 lp[GATED_PPL];
+#pragma unroll
+                for (int j = 0; j < GATED_PPL; ++j) {
+                    const u32 r = j * WAVE + lane;
+                    bool on = r < m;
+                    if (dense) {
+                        lp[j] = q * (WAVE * 32) + n + r;
+                        on = (words[w][lp[j] >> 5] >> (lane & 31)) & 1u;
+                    } else {
+                        lp[j] = on ? list[w][n + r] : 0u;
+                    }
+                    // dense: the tokens are loaded whatever the bit says, a wave's in a row
+                    u32 nxt = SENT;
+                    u64 ck = EMPTY;
+                    if ((dense || on) && p00 + lp[j] < L) ck = ctx_key_at<K>(tok, p00 + lp[j], k, nxt);
+                    wk[j].key = on && nxt != SENT ? ck : EMPTY;
+                    wk[j].next = nxt;
+                }
+#pragma unroll
+                for (int j = 0; j < GATED_PPL; ++j) walk_seed2(vt, vcap, wk[j].key, wk[j].next, wk[j]);
+#pragma unroll
+                for (int j = 0; j < GATED_PPL; ++j) {
+                    if (j * WAVE >= m) break;  // wave-uniform
+                    const u64 hk = walk_end2<K>(tok, p00 + lp[j], k, vt, vrep, x, flags, wk[j]);
+                    const bool hit = hk != EMPTY;
+                    const u64 b = __ballot(hit);
+                    if (dense) {
+                        if ((lane & 31) == 0) words[w][lp[j] >> 5] = lane ? (u32)(b >> 32) : (u32)b;
+                    } else if (hit) {
+                        atomicOr(&words[w][lp[j] >> 5], 1u << (lp[j] & 31));
+                    }
+                    if constexpr (S::KIND == 2) emit_wave(sink, &ss, b, hit, hk, p00 + lp[j], flags);
+                    else if (hit) sink_hit(sink, hk, p00 + lp[j], full, flags);
+                }
+            }
+        }
+        for (int q = 0; q < ng; ++q) {
+            const i64 wi = (g0 + q) * WAVE + lane;
+            if (wi < nwords) bm_out[wi] = words[w][q * WAVE + lane];
+        }
+    }
+    sink_end(sink, &ss);
+}
+
 // A bitmap's set bits listed in two passes over blocks of up to BL_ROUNDS rounds of BL_BLOCK words (fewer rounds for
 // a small bitmap, so that it still spreads over about 1024 blocks): each block's count, a scan of those counts, then
 // each block lists its bits in order (a round of BL_BLOCK words at a time, their offsets by a block-wide scan), so no
@@ -428,13 +558,16 @@ static void fill_u32_n(u32* p, u32 v, i64 n, hipStream_t st) {
     if (n > 0) fill_u32_small_k<<<grid_for(n, 256), 256, 0, st>>>(p, v, n);
 }
 
-// One level scan with a sink: sparse 0 a lane per position, 1 a lane per bitmap word, 2 LDS-listed (bm_in required
-// for 1 and 2).
+// One level scan with a sink: sparse 0 a lane per position, 1 a lane per bitmap word, 2 LDS-listed, 4 either of 0 and 2
+// by each span's own density (bm_in required for 1, 2 and 4).
 template <class S>
 static int launch_scan(const u16* tok, i64 L, int k, const u32* bm_in, u32* bm_out, const u64* vt, u64 vcap,
                         const u32* vrep, const u16* x, const S& sink, u32* flags, int grid, int sparse, hipStream_t st,
                         const u32* pre = nullptr) {
-    if (sparse == 2 && bm_in) {
+    if (sparse == 4 && bm_in) {
+        LEVEL_DISPATCH(k, (scan_gated_k<K, S><<<grid, 256, 0, st>>>(tok, L, k, bm_in, bm_out, vt, vcap, vrep, x, sink, flags,
+                                                                   pre)));
+    } else if (sparse == 2 && bm_in) {
         LEVEL_DISPATCH(k, (scan_compact_k<K, S><<<grid, 256, 0, st>>>(tok, L, k, bm_in, bm_out, vt, vcap, vrep, x, sink, flags,
                                                                      pre)));
     } else if (sparse && bm_in) {

@@ -315,11 +315,14 @@ class LevelBuild:
     def _mode(self, si: int, scanned: list) -> int:
         """A shard's si-th scanned level's scan: a lane per position (0) for the first level and behind a dense
         previous level, the LDS-listed set positions (2) behind a sparser one, or below LIST_DENSITY the set positions
-        listed in memory first (3). Densities are the last build's (dense when unknown)."""
+        listed in memory first (3). Densities are those of a build that read hit statistics; without them each wave
+        decides for its own positions (4)."""
         if si == 0:
             return 0
         d = self.density.get(scanned[si - 1])
-        if d is None or d >= 0.5:
+        if d is None:
+            return 4
+        if d >= 0.5:
             return 0
         return 3 if d < LIST_DENSITY else 2
 
