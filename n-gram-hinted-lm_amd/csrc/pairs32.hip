@@ -571,12 +571,18 @@ __device__ __forceinline__ void agg_clear(int nid, u32* s_tot, u32* s_dist, u64*
     for (int l = threadIdx.x; l < nid * KT; l += AGG_BLOCK) s_top[l] = 0;
 }
 
-// *present += the block's present contexts (one atomic per wave).
-__device__ __forceinline__ void agg_present(u32 mine, u64* present) {
+// *present += the block's present contexts: its waves' sums met in LDS (s_sum, a word no one else uses any more), then
+// one atomic per block (same-address atomics run at about 80 M/s: one per wave cost a block per group of ids 5 ms).
+__device__ __forceinline__ void agg_present(u32 mine, u64* present, u32* s_sum) {
     u32 sm = mine;
 #pragma unroll
     for (int d = WAVE / 2; d > 0; d >>= 1) sm += (u32)__shfl_down((int)sm, d, WAVE);
-    if (lane_id() == 0 && sm) atomicAdd((unsigned long long*)present, (unsigned long long)sm);
+    __syncthreads();
+    if (threadIdx.x == 0) *s_sum = 0;
+    __syncthreads();
+    if (lane_id() == 0 && sm) atomicAdd(s_sum, sm);
+    __syncthreads();
+    if (threadIdx.x == 0 && *s_sum) atomicAdd((unsigned long long*)present, (unsigned long long)*s_sum);
 }
 
 // Two blocks share a compute unit where the LDS allows (KT <= 4: 80 KB each): 8 waves per SIMD, so at most 96
@@ -636,7 +642,7 @@ __global__ void __launch_bounds__(AGG_BLOCK) __attribute__((amdgpu_waves_per_eu(
             nwe = start[q + gridDim.x + 1];
         }
     }
-    if (present) agg_present(mine, present);
+    if (present) agg_present(mine, present, s_tot);
 }
 
 // ctx_agg_k over ng_part_count32's words left in runs (its `runs` mode, events keyed by kmix(pair key, W, W - d1)):
@@ -730,7 +736,7 @@ __global__ void __launch_bounds__(AGG_BLOCK) __attribute__((amdgpu_waves_per_eu(
         mine += agg_flush<KT>(lo, nid, n_ids, s_tot, s_dist, s_top, rec, dist, 0, nullptr, 0, nullptr);
         lds_barrier();  // the LDS is read before the next group clears it
     }
-    if (present) agg_present(mine, present);
+    if (present) agg_present(mine, present, s_tot);
 }
 
 static inline int grid_cap(i64 n, int cap) { return n < 1 ? 1 : n > cap ? cap : (int)n; }

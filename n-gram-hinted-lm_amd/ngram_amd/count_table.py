@@ -206,7 +206,8 @@ class CountTable:
         min_pbits = 0
         while True:
             c = P.count32(lib, seg, ccap, TOPE, None, n_k, self.ratio.get(k, 1.0), ev_name, min_pbits, slabs=True,
-                          deep_min=CNT_TOP, with_dist=False, agg_grid=self.grid // EMIT_BLOCKS_PER_CU * 2)
+                          deep_min=CNT_TOP, with_dist=False, agg_grid=self.grid // EMIT_BLOCKS_PER_CU * 2,
+                          count_present=True)
             st = torch.cat([c.stat, c.deep_n]).cpu().tolist()  # one host read: totals, flags, deep contexts
             if int(st[2]) & 1 and c.pbits < P.pbits32_max(ccap):  # a partition overfull: count with a bit more
                 min_pbits = c.pbits + 1

@@ -328,7 +328,7 @@ def pbits32_max(n_ids: int) -> int:
 def count32(elib: Lib, seg: tuple, n_ids: int, ktop: int, lookups: tuple | None, n_events: int | None,
             ratio: float = 1.0, event=_no_event, min_pbits: int = 0, slabs: bool = False,
             deep_min: int | None = None, with_dist: bool = True, agg_grid: int = 0,
-            stat: torch.Tensor | None = None, mbits: int | None = None) -> Counted32:
+            stat: torch.Tensor | None = None, mbits: int | None = None, count_present: bool = False) -> Counted32:
     """Count a level's events emitted by ng_scan_emit in the W-bit mode (wbits = W = w_bits(n_ids)[1], dbits =
     first_digit(W); seg = (regions, R, ev_count, dhist, nseg, scan flags)) and make every present context's record
     (top ktop) without a host read: the passes and the count of pairs32.hip. `n_events`: the level's events (the last
@@ -468,7 +468,7 @@ def count32(elib: Lib, seg: tuple, n_ids: int, ktop: int, lookups: tuple | None,
     e0.record()
     elib("ng_ctx_agg", words, start2, P2, i32(ibits), i32(cb), n_ids, esc_k, esc_c, u64(ESC_CAP), i32(ktop), rec,
          dist, flags, ctypes.c_uint32(deep_min or 0), deep, u64(deep.numel() if deep is not None else 0), deep_n,
-         deep_n[1:] if deep_n is not None else None, i32(agg_grid))
+         deep_n[1:] if count_present else None, i32(agg_grid))
     e1.record()
     keep = deep_min is not None
     return Counted32(rec, dist, qcnt, stat, pbits, cb, (esc_k, esc_c), W, slab, words if keep else None,
