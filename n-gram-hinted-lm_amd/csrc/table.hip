@@ -383,7 +383,9 @@ extern "C" int ng_ctx_kth_grouped(const u64* w, const i64* gstart, int ibits, in
                                   u64* thr, void* stream) {
     if (kth < 1 || cb <= 0 || cb > 44 || esc_cap == 0 || gstart == nullptr || ibits < 0 || ibits > 11) return -1;
     if (m > 0) {
-        const int g = m < 65536 ? (int)m : 65536;
+        // with a device-side count, m only bounds it (by the pairs, far above the contexts that have kth of them)
+        const int most = m_dev ? 2048 : 65536;
+        const int g = m < most ? (int)m : most;
         ctx_kth_k<<<g, 256, 0, (hipStream_t)stream>>>(w, cb, esc_k, esc_c, esc_cap, nullptr, ids, m, kth, thr, gstart,
                                                       ibits, m_dev);
     }

@@ -15,9 +15,9 @@ counted with global atomics in one hash table and ranked by a second sort; here
      position the rule drops is a request saved;
   3. the events are hash-partitioned by a radix pass straight from the regions and counted partition by partition in
      LDS (partcount.count_events), which also answers each query position's (context, target) count;
-  4. the distinct pairs, packed one word each, are sorted by context and summarized per present context
-     (ng_ctx_summary: total, pairs, top entries); with a TOP rule the contexts with more than `cnt_top` pairs get the
-     cnt_top-th largest score (ng_ctx_kth);
+  4. the distinct pairs, packed one word each, are summarized per present context (total, pairs, top entries); with a
+     TOP rule the contexts with more than `cnt_top` pairs get the cnt_top-th largest score (ng_ctx_kth_grouped; on the
+     64-bit path ng_ctx_kth);
   5. per query position its context's record gives tot, dist, the target's count (if ranked within cnt_top) and the
      top entries (ng_pos_summary), and the level's mask bit.
 
@@ -154,7 +154,7 @@ class LevelBuild:
             seen = seen_n = None
             seen_cap = 0
             if prev is not None and self.level_shards[k] <= self.level_shards[prev]:
-                if cnt_top is None and k not in self.wide and k in self.seen_of and _defer:
+                if k not in self.wide and k in self.seen_of and _defer:
                     # listed on the device, sized from the last build's count: no host wait (checked after the last
                     # level; a list that came out longer than its room makes the build run again)
                     seen_cap = min(N, int(self.seen_of[k] * max(SEEN_MARGIN, 1.0)) + 4096)
@@ -166,7 +166,7 @@ class LevelBuild:
                     seen = torch.nonzero(out[1, li - 1] > 0).squeeze(1).to(torch.int32)
                     self.seen_of[k] = int(seen.numel())
             kept = k in keep
-            ktop = 8 if (kept or cnt_top is not None) else _record_width(topk)
+            ktop = 8 if kept else _record_width(topk)
             q0, q1 = self._event("qindex", k, N)
             q0.record()
             vi = QueryIndex(elib, x, avail, k, seen, expect=self.contexts_of.get(k), defer=_defer, n_dev=seen_n,
@@ -179,11 +179,17 @@ class LevelBuild:
             t1 = time.perf_counter()
             ev_fn = lambda name, n, k=k: self._event(name, k, n)  # noqa: E731
             _, W = w_bits(vi.ids)
-            use32 = cnt_top is None and W <= W_MAX and k not in self.wide
+            # with a TOP rule the 64-bit count still takes what the 32-bit one does not: no shards, or regions of 2^32
+            # events or more (its offsets are 32-bit; the events themselves may be fewer)
+            use32 = W <= W_MAX and k not in self.wide and \
+                (cnt_top is None or (self.level_shards[k] > 0 and n_reg < 1 << 32))
             if not use32 and seen_n is not None:  # the 64-bit count takes an exact list: read its length
                 seen = seen[: int(seen_n.item())]
                 seen_n = None
-            mbits = self._mbits(W, vi.ids, ktop) if use32 else 0
+            if not use32 and cnt_top is not None:
+                ktop = 8  # its thresholds find a context's words by its record's first word, which top 8 has room for
+            # with a TOP rule the words are grouped by context, for the thresholds: no runs
+            mbits = 0 if not use32 else W if cnt_top is not None else self._mbits(W, vi.ids, ktop)
             seg = self._emit(k, vi, x, bms, regions, R, W if use32 else 0,
                              stats[li, 3:4].view(torch.int32) if use32 else None, mbits)
             t2 = time.perf_counter()
@@ -191,7 +197,7 @@ class LevelBuild:
                 # the 32-bit count: records made without sorting the pairs, every size read once after the last level
                 c = count32(elib, seg, vi.ids, ktop, (vi.ctx_of, tgt, seen, seen_n), self.events_of.get(k),
                             self.dratio.get(k, 1.0), ev_fn, self.min_pbits.get(k, 0), stat=stats[li],
-                            mbits=mbits)
+                            mbits=mbits, deep_min=cnt_top)
                 del seg
                 checks32.append((k, li, c.pbits, vi.ids, seen_cap if seen_n is not None else -1))
                 sm = c
@@ -218,8 +224,12 @@ class LevelBuild:
                 thr = elib.zeros(vi.ids, torch.int64, dev)
                 e0, e1 = self._event("ctx_kth", k, int(sm.deep.numel()))
                 e0.record()
-                elib("ng_ctx_kth", sm.words, i32(c.cb), c.esc[0], c.esc[1], u64(partcount.ESC_CAP), sm.rec, sm.deep,
-                     sm.deep.numel(), i32(cnt_top), thr)
+                if use32:  # how many there are stays on the device
+                    elib("ng_ctx_kth_grouped", c.words, c.wstart, i32(c.ibits), i32(c.cb), c.esc[0], c.esc[1],
+                         u64(partcount.ESC_CAP), c.deep, c.deep.numel(), c.deep_n, i32(cnt_top), thr)
+                else:
+                    elib("ng_ctx_kth", sm.words, i32(c.cb), c.esc[0], c.esc[1], u64(partcount.ESC_CAP), sm.rec,
+                         sm.deep, sm.deep.numel(), i32(cnt_top), thr)
                 e1.record()
             e0, e1 = self._event("pos_gather", k, N)
             e0.record()
