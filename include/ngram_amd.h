@@ -385,6 +385,19 @@ int ng_table_query32(const uint16_t* x, const int* avail, const uint16_t* tgt, n
 /* hint rows over table levels (count_table.rs query_rows :338-404); desc[v * 3]: slot_of, records, bucket */
 int ng_pos_rows(ng_i64 N, int nlv, const ng_i64* desc, int entries, short* cell, uint16_t* next, uint16_t* weights,
                 signed char* level, void* stream);
+/* an online stream's layout and training order, made on the device: tau / tau_in (first step training a position as an
+ * input or a span's last target / as an input; 2^32 - 1: none) from spans [m, 3] (lo, hi, step), offs [m + 1] their
+ * lengths' exclusive sums (total = offs[m]); start[g] (g at a part's first token or a BOS, else 0) and has_next[g];
+ * avail from each position's segment start; the positions' sort keys by step (k 0: tau[g], else 1 + the largest tau of
+ * the k-context occurrence ending at g and its next token; `none` where there is none), val[g] = g. bounds: the np
+ * parts' starts, then n */
+int ng_online_tau(const ng_i64* spans, const ng_i64* offs, ng_i64 m, ng_i64 total, const ng_i64* bounds, ng_i64 np,
+                  ng_i64 n, uint32_t* tau, uint32_t* tau_in, void* stream);
+int ng_online_layout(const uint16_t* tok, ng_i64 n, const ng_i64* bounds, ng_i64 np, ng_i64* start,
+                     unsigned char* has_next, void* stream);
+int ng_online_avail(const ng_i64* seg, ng_i64 n, int* avail, void* stream);
+int ng_online_order(const uint32_t* tau, ng_i64 n, const ng_i64* bounds, ng_i64 np, int k, ng_u64 none, ng_u64* key,
+                    uint32_t* val, void* stream);
 /* online state (online.rs step rule), per level: a context table ck (slot = context id); a pair table pt of pcap
  * 16-byte slots (pt[2s] the key slot << 16 | next, EMPTY when free; the low half of pt[2s + 1] its count); a record
  * per context, rw u32 words: [0] total, [1] distinct next tokens, and with rw = 16 (levels with hint rows) [2, 10) the

@@ -21,7 +21,6 @@ import ctypes
 import numpy as np
 import torch
 
-from .data import BOS
 from .lib import Lib, i32, u64
 
 
@@ -94,21 +93,23 @@ def plan_rows(plan: np.ndarray, sizes: list[int], BT: int, accum: int, rank: int
     return rows
 
 
-def _tau(n: int, bounds: list[int], spans: np.ndarray) -> tuple[np.ndarray, np.ndarray]:
-    """tau (first step training a position as an input or a target) and tau_in (as an input) (online.rs:137-158)."""
-    tau = np.full(n, NONE, np.uint64)
-    tau_in = np.full(n, NONE, np.uint64)
-    b = np.asarray(bounds, np.int64)
-    sp = np.asarray(spans, np.int64).reshape(-1, 3)
-    order = np.argsort(sp[:, 2], kind="stable")[::-1]  # larger steps first: smaller ones overwrite (a minimum)
-    for lo, hi, step in sp[order]:
-        tau[lo:hi] = np.minimum(tau[lo:hi], step)
-        tau_in[lo:hi] = np.minimum(tau_in[lo:hi], step)
-        if hi > lo and hi < n:
-            part = int(np.searchsorted(b, hi - 1, side="right"))
-            if hi < b[part]:
-                tau[hi] = min(int(tau[hi]), int(step))
-    return tau, tau_in
+STEP_TABLE = 1 << 20  # up to this many steps their list's bounds are looked up for every step, else for the ones in use
+
+
+class _Steps:
+    """A list ordered by step, as its bounds: `steps` (ascending, int64) and where each of them begins; entries of a
+    step that is not among them: none."""
+
+    def __init__(self, steps: np.ndarray, begins: np.ndarray, total: int):
+        self.steps = steps
+        self.begins = np.append(begins, total)
+
+    def before(self, s: int) -> int:
+        """The entries of the steps before s."""
+        return int(self.begins[np.searchsorted(self.steps, s, side="left")])
+
+    def sizes(self) -> np.ndarray:
+        return np.diff(self.begins)
 
 
 class OnlineRows:
@@ -134,20 +135,24 @@ class OnlineRows:
         self.lib = Lib()
         dev = torch.device("cuda", torch.cuda.current_device())
         self.dev = dev
-        self.tok = torch.from_numpy(tok.view(np.int16).copy()).to(dev)
-        tau, tau_in = _tau(n, bounds, sp)
-        self.tau = torch.from_numpy(tau.astype(np.int64)).to(dev)
-        self.tau_in = torch.from_numpy(tau_in.astype(np.int64)).to(dev)
-        # segments (start at each part and at every BOS), the next token's part, each position's part bounds
-        idx = torch.arange(n, device=dev)
-        part_of = torch.bucketize(idx, torch.tensor(bounds[1:], device=dev), right=True)
-        bt = torch.tensor(bounds, device=dev)
-        self.part_lo, self.part_hi = bt[part_of], bt[part_of + 1]
-        start = ((self.tok.to(torch.int32) & 0xFFFF) == BOS) | (idx == self.part_lo)
-        seg = torch.cummax(torch.where(start, idx, torch.zeros_like(idx)), 0).values
-        self.avail = (idx - seg + 1).to(torch.int32)
-        self.seg_index = torch.cumsum(start.to(torch.int64), 0) - 1  # the rule "segment"'s steps
-        self.has_next = (idx + 1 < self.part_hi).to(torch.uint8)
+        self.tok = torch.from_numpy(tok.view(np.int16) if tok.flags.writeable else tok.view(np.int16).copy()).to(dev)
+        # the first step training each position (as an input or a target; as an input), its segment and whether its next
+        # token lies in its part, on the device (uint32 bits, NONE where no step does)
+        self.bounds_dev = torch.tensor(bounds, dtype=torch.int64, device=dev)
+        np_ = len(bounds) - 1
+        offs = np.concatenate([[0], np.cumsum(sp[:, 1] - sp[:, 0])]).astype(np.int64)
+        at = torch.from_numpy(np.concatenate([sp.reshape(-1), offs])).to(dev)
+        self.tau = torch.empty(n, dtype=torch.int32, device=dev)
+        self.tau_in = torch.empty(n, dtype=torch.int32, device=dev)
+        self.lib("ng_online_tau", at, at[sp.size :], len(sp), int(offs[-1]), self.bounds_dev, np_, n, self.tau,
+                 self.tau_in)
+        self.max_step = int(sp[:, 2].max()) if len(sp) else -1
+        seg = torch.empty(n, dtype=torch.int64, device=dev)
+        self.has_next = torch.empty(n, dtype=torch.uint8, device=dev)
+        self.lib("ng_online_layout", self.tok, n, self.bounds_dev, np_, seg, self.has_next)
+        self.lib.cub("inclusive_max", seg, seg, n)
+        self.avail = torch.empty(n, dtype=torch.int32, device=dev)
+        self.lib("ng_online_avail", seg, n, self.avail)
         self._done = 0
         self.config = None
         self.state = None
@@ -190,34 +195,18 @@ class OnlineRows:
         self.state = self._new_state(cfg)
 
     def _new_state(self, cfg, taus=None) -> dict:
-        """advance()'s state; taus: (tau, tau_in) in place of the spans' (the rule "segment"'s)."""
+        """advance()'s state; taus: (tau, tau_in, the last step) in place of the spans' (the rule "segment"'s)."""
         levels, buckets, entries, count_levels = cfg
-        dev, n = self.dev, self.n
-        tau_all, tau_in_all = taus if taus is not None else (self.tau, self.tau_in)
+        dev = self.dev
+        tau, tau_in, last = taus if taus is not None else (self.tau, self.tau_in, self.max_step)
         E = max(1, entries)
         st = {"levels": {}, "E": E}
-        # queries: positions trained as inputs, by step
-        q_valid = tau_in_all != NONE
-        q_pos = torch.nonzero(q_valid).squeeze(1)
-        q_step = tau_in_all[q_pos]
-        order = torch.sort(q_step, stable=True).indices
-        st["q_pos"] = q_pos[order].to(torch.int32).contiguous()
-        st["q_step"] = q_step[order].cpu().numpy()
-        idx = torch.arange(n, device=dev)
-        for k in sorted(set(levels) | set(count_levels)):
-            # occurrences ending at g: tokens g-k+1..g and next g+1 within g's part; alpha = 1 + max tau over them
-            ok = (idx - k + 1 >= self.part_lo) & (idx + 1 < self.part_hi)
-            a = torch.full((n,), -1, dtype=torch.int64, device=dev)
-            for d in range(-k + 1, 2):
-                sh = torch.full((n,), NONE, dtype=torch.int64, device=dev)
-                lo, hi = max(0, -d), min(n, n - d)
-                if hi > lo:
-                    sh[lo:hi] = tau_all[lo + d : hi + d]
-                a = torch.maximum(a, sh)
-            ok &= a != NONE
-            occ = torch.nonzero(ok).squeeze(1)
-            alpha = a[occ] + 1
-            o = torch.sort(alpha, stable=True).indices
+        # queries: the positions trained as inputs, by step; and per level its occurrences (ending at g: tokens g-k+1..g
+        # and next g+1 within g's part) by the step they count from, alpha = 1 + max tau over them
+        ks = sorted(set(levels) | set(count_levels))
+        orders = self._by_step([(tau_in, 0)] + [(tau, k) for k in ks], last + 1)
+        st["q_pos"], st["q_step"] = orders[0]
+        for k, (occ, alpha) in zip(ks, orders[1:]):
             m = int(occ.numel())
             cap = max(1 << 16, int(m / LOAD) + 1)
             # the pair table: 16-byte slots (key, count); a record per context: total, distinct count and, where the
@@ -226,7 +215,7 @@ class OnlineRows:
             pt[:, 1] = 0
             rw = REC_TOP if k in levels else REC_CNT
             st["levels"][k] = {
-                "occ": occ[o].to(torch.int32).contiguous(), "alpha": alpha[o].cpu().numpy(),
+                "occ": occ, "alpha": alpha,
                 "ck": torch.full((cap,), -1, dtype=torch.int64, device=dev), "ccap": cap,
                 "pt": pt, "pcap": cap, "rec": torch.zeros(cap * rw, dtype=torch.int32, device=dev), "rw": rw,
                 "flags": torch.zeros(2, dtype=torch.int32, device=dev),
@@ -243,14 +232,7 @@ class OnlineRows:
             desc += [lv["pt"].data_ptr(), lv["pcap"], lv["rec"].data_ptr(), int(lv["rw"] == REC_TOP),
                      lv["flags"].data_ptr()]
         st["top_desc"] = torch.tensor(desc, dtype=torch.int64, device=dev)
-        per_step = np.zeros(1, np.int64)
-        for lv in st["levels"].values():
-            if len(lv["alpha"]):
-                c = np.bincount(lv["alpha"])
-                if len(c) > len(per_step):
-                    per_step = np.pad(per_step, (0, len(c) - len(per_step)))
-                per_step[: len(c)] += c
-        most = max(1, int(per_step.max()))
+        most = max(1, self._most(lv["alpha"] for lv in st["levels"].values()))
         st["ev"] = torch.empty(most, dtype=torch.int64, device=dev)
         st["merge_temp"] = None
         if self.merge == "buckets":
@@ -269,7 +251,7 @@ class OnlineRows:
             st["agg"] = torch.empty(most, dtype=torch.int32, device=dev)
             st["nruns"] = torch.zeros(1, dtype=torch.int64, device=dev)
             st["score"] = torch.empty(most, dtype=torch.int64, device=dev)
-        nq = int(np.bincount(st["q_step"]).max()) if len(st["q_step"]) else 1
+        nq = self._most([st["q_step"]])
         st["qslot"] = {k: torch.empty(max(1, nq), dtype=torch.int32, device=dev) for k in levels}
         st["hinted"] = torch.zeros(1, dtype=torch.int32, device=dev)
         st["done"] = 0
@@ -281,8 +263,47 @@ class OnlineRows:
             st["rows_desc"] = torch.tensor(desc, dtype=torch.int64, device=dev)
         return st
 
-    def _range(self, arr: np.ndarray, lo: int, hi: int) -> tuple[int, int]:
-        return int(np.searchsorted(arr, lo, side="left")), int(np.searchsorted(arr, hi, side="left"))
+    def _by_step(self, lists: list, last: int) -> list:
+        """Per (tau, k) of `lists` the positions with a step, ordered by it and within a step by position (int32), and
+        the steps' bounds (ng_online_order's steps, at most `last`; a stable sort by them)."""
+        n, dev = self.n, self.dev
+        bits = max(1, (last + 1).bit_length())
+        none = (1 << bits) - 1  # above every step: the positions without one sort behind the others
+        table = last < STEP_TABLE
+        steps = torch.arange(last + 2, device=dev) if table else None
+        key, key2 = (torch.empty(n, dtype=torch.int64, device=dev) for _ in range(2))
+        val = torch.empty(n, dtype=torch.int32, device=dev)
+        out, bounds = [], []
+        for tau, k in lists:
+            order = torch.empty(n, dtype=torch.int32, device=dev)
+            self.lib("ng_online_order", tau, n, self.bounds_dev, len(self.bounds) - 1, i32(k), u64(none), key, val)
+            self.lib.cub("sort_pairs", key, key2, val, order, n, i32(0), i32(bits))
+            out.append(order)
+            if table:
+                bounds.append(torch.searchsorted(key2, steps))
+            else:
+                u, c = torch.unique_consecutive(key2, return_counts=True)
+                u, c = u.cpu().numpy(), c.cpu().numpy()
+                begins = np.cumsum(c) - c
+                at = int(np.searchsorted(u, none))
+                bounds.append(_Steps(u[:at], begins[:at], int(begins[at]) if at < len(u) else n))
+        if table:
+            host = torch.stack(bounds).cpu().numpy()  # one read for every list
+            bounds = [_Steps(np.arange(last + 1), h[:-1], int(h[-1])) for h in host]
+        return [(order[: int(b.begins[-1])], b) for order, b in zip(out, bounds)]
+
+    @staticmethod
+    def _most(lists) -> int:
+        """The most entries one step has in all of `lists` together."""
+        lists = list(lists)
+        steps = np.unique(np.concatenate([b.steps for b in lists])) if lists else np.zeros(0, np.int64)
+        total = np.zeros(len(steps), np.int64)
+        for b in lists:
+            total[np.searchsorted(steps, b.steps)] += b.sizes()
+        return int(total.max()) if len(total) else 0
+
+    def _range(self, steps: _Steps, lo: int, hi: int) -> tuple[int, int]:
+        return steps.before(lo), steps.before(hi)
 
     def _step(self, st: dict, s: int, outs: dict, queries: bool = True) -> None:
         """Step s: its newly available occurrences inserted at every level, then (queries) its queries answered."""
@@ -413,8 +434,10 @@ class OnlineRows:
         query exactly when that segment lies before the query's; every step then runs as advance()'s do."""
         taus = None
         if rule == "segment":
-            taus = (self.seg_index, self.seg_index)
-            step_lo, step_hi = 0, int(self.seg_index[-1].item()) + 1
+            seg = (torch.cumsum(self.avail == 1, 0) - 1).to(torch.int32)  # a segment starts where avail is 1
+            last = int(seg[-1].item())
+            taus = (seg, seg, last)
+            step_lo, step_hi = 0, last + 1
         elif rule != "step":
             raise ValueError(f"rule must be 'step' or 'segment': {rule}")
         if step_lo > step_hi or step_hi >= 1 << 30:

@@ -1,0 +1,54 @@
+"""GPU: an online stream's layout and training order made on the device (ng_online_tau, ng_online_layout,
+ng_online_avail, ng_online_order and a stable sort), against a position-by-position restatement: overlapping, empty and
+out-of-order spans, parts and end-of-text tokens, contexts longer than a part, steps close together and far apart."""
+
+import numpy as np
+import pytest
+
+from ngram_amd.online import NONE, OnlineRows
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,parts", [(1, 1), (2, 2), (17, 3), (300, 1), (5000, 7)])
+@pytest.mark.parametrize("spread", [1, 40_000_000])
+def test_training_order(gpu, n, parts, spread):
+    rng = np.random.default_rng(n + parts)
+    tok = rng.integers(0, 50, n).astype(np.uint16)
+    tok[rng.random(n) < 0.05] = 50256
+    bounds = [0, *sorted(rng.choice(np.arange(1, n), parts - 1, replace=False).tolist()), n] if parts > 1 else [0, n]
+    lo = rng.integers(0, n + 1, 3 * parts)
+    hi = np.minimum(lo + rng.integers(0, max(2, n // 4), 3 * parts), n)
+    spans = np.stack([lo, hi, rng.integers(0, 9, 3 * parts) * spread], 1)
+    rows = OnlineRows(tok, bounds, spans)
+    tau, tau_in = np.full(n, NONE, np.int64), np.full(n, NONE, np.int64)
+    part = np.searchsorted(bounds, np.arange(n), side="right") - 1
+    for a, b, s in spans:
+        tau_in[a:b] = np.minimum(tau_in[a:b], s)
+        tau[a:b] = np.minimum(tau[a:b], s)
+        if b > a and b < n and part[b] == part[b - 1]:
+            tau[b] = min(tau[b], s)
+    assert np.array_equal(rows.tau.cpu().numpy().view(np.uint32), tau)
+    assert np.array_equal(rows.tau_in.cpu().numpy().view(np.uint32), tau_in)
+    avail, has_next = np.zeros(n, np.int64), np.zeros(n, np.int64)
+    for g in range(n):
+        avail[g] = 1 if tok[g] == 50256 or g == bounds[part[g]] else avail[g - 1] + 1
+        has_next[g] = g + 1 < n and part[g + 1] == part[g]
+    assert np.array_equal(rows.avail.cpu().numpy(), avail)
+    assert np.array_equal(rows.has_next.cpu().numpy(), has_next)
+    levels = [1, 2, 5, 20]
+    got = rows._by_step([(rows.tau_in, 0)] + [(rows.tau, k) for k in levels], rows.max_step + 1)
+    for (order, steps), k in zip(got, [0, *levels]):
+        if k == 0:
+            step = tau_in
+        else:
+            step = np.full(n, NONE, np.int64)
+            for g in range(n):
+                if g - k + 1 >= bounds[part[g]] and has_next[g]:
+                    m = tau[g - k + 1 : g + 2].max()
+                    step[g] = m + 1 if m != NONE else NONE
+        want = np.flatnonzero(step != NONE)
+        want = want[np.argsort(step[want], kind="stable")]
+        assert np.array_equal(order.cpu().numpy(), want), k
+        for s in {0, 1, int(spread), int(spans[:, 2].max()) + 1, *step[want].tolist()}:
+            assert steps.before(int(s)) == int((step[want] < s).sum()), (k, s)
