@@ -398,6 +398,21 @@ int ng_online_layout(const uint16_t* tok, ng_i64 n, const ng_i64* bounds, ng_i64
 int ng_online_avail(const ng_i64* seg, ng_i64 n, int* avail, void* stream);
 int ng_online_order(const uint32_t* tau, ng_i64 n, const ng_i64* bounds, ng_i64 np, int k, ng_u64 none, ng_u64* key,
                     uint32_t* val, void* stream);
+/* the count rows of a range of steps at once (online.rs :259 counts): a level's occurrences in the order of their steps
+ * (ng_online_order's keys akey and positions occ, sorted) inserted into the context table ck (ccap < 2^cbits slots,
+ * EMPTY-filled), key[i] = slot << 16 | next (all ones of 16 + cbits bits: none), val[i] = i; from those sorted stably by
+ * bits [0, 16 + cbits) (ka, va) and [16, 16 + cbits) (kb, vb) each context's bounds (2 u32 per slot) and the sums pre
+ * (n + 1 u32) of pairs' first occurrences (first: n bytes of scratch; two-phase temp storage); then tot / dist / cnt of
+ * the queries pos[0..m) (NULL: 0..m - 1) of step[g] into row g, column ci of [.., nc] arrays; flags[0] bit 1: ck full */
+int ng_online_occ_insert(const uint16_t* tok, const uint32_t* occ, const ng_u64* akey, ng_u64 none, ng_i64 n, int k,
+                         ng_u64* ck, ng_u64 ccap, int cbits, ng_u64* key, uint32_t* val, uint32_t* flags, void* stream);
+int ng_online_occ_index(void* temp, size_t* temp_bytes, const ng_u64* ka, const uint32_t* va, const ng_u64* kb,
+                        const uint32_t* vb, ng_i64 n, int cbits, unsigned char* first, uint32_t* pre, uint32_t* bounds,
+                        void* stream);
+int ng_online_occ_query(const uint16_t* tok, const int* avail, const unsigned char* has_next, const int* pos, ng_i64 m,
+                        const uint32_t* step, const ng_u64* akey, ng_i64 n, int k, const ng_u64* ck, ng_u64 ccap,
+                        const uint32_t* bounds, const uint32_t* vb, const uint32_t* pre, const ng_u64* ka,
+                        const uint32_t* va, uint32_t* tot, uint16_t* dist, uint32_t* cnt, int nc, int ci, void* stream);
 /* online state (online.rs step rule), per level: a context table ck (slot = context id); a pair table pt of pcap
  * 16-byte slots (pt[2s] the key slot << 16 | next, EMPTY when free; the low half of pt[2s + 1] its count); a record
  * per context, rw u32 words: [0] total, [1] distinct next tokens, and with rw = 16 (levels with hint rows) [2, 10) the

@@ -11,8 +11,8 @@ a query's k-context must lie in its segment (segments start at each part's start
 totals, distinct counts and exact top-`entries` lists, and a split pair table) persists between calls; a step inserts
 its newly available occurrences, then answers its queries (libngram_amd.so: ng_online_insert_levels, sort_pairs,
 reduce_by_key, ng_online_top, ng_online_query_levels, ng_online_rows). `hints` / `counts` answer a step range from a fresh
-state; with rule="segment" (the reference's exactness-test rule) they answer every position from its segment's
-start, one step per segment."""
+state (counts alone need none: every step at once, online_counts.hip); with rule="segment" (the reference's
+exactness-test rule) they answer every position from its segment's start, a step per segment."""
 
 from __future__ import annotations
 
@@ -425,13 +425,8 @@ class OnlineRows:
             self._step(st, s, outs)
         self._done = step_hi
 
-    def _range_rows(self, levels, buckets, entries, count_levels, step_lo, step_hi, rule, slots: int = 1,
-                    with_level: bool = False):
-        """A fresh state advanced over steps [0, step_hi), the queries of [step_lo, step_hi) answered. The rule
-        "segment" (online.rs:14-17: every position a query at its segment's start, an occurrence counted iff its next
-        token lies before that start) is the step rule with one step per segment in stream order: tau = tau_in = the
-        position's segment index makes an occurrence's alpha 1 + the segment of its next token, so it counts for a
-        query exactly when that segment lies before the query's; every step then runs as advance()'s do."""
+    def _rule(self, rule: str, step_lo: int, step_hi: int) -> tuple:
+        """(tau, tau_in, the last step), or None for the spans', and the step range of a rule."""
         taus = None
         if rule == "segment":
             seg = (torch.cumsum(self.avail == 1, 0) - 1).to(torch.int32)  # a segment starts where avail is 1
@@ -442,6 +437,65 @@ class OnlineRows:
             raise ValueError(f"rule must be 'step' or 'segment': {rule}")
         if step_lo > step_hi or step_hi >= 1 << 30:
             raise ValueError(f"bad step range [{step_lo}, {step_hi})")
+        return taus, step_lo, step_hi
+
+    def _range_counts(self, count_levels, step_lo, step_hi, rule):
+        """The count rows of the queries of [step_lo, step_hi) (outputs and positions as _range_rows'), every step at once:
+        per level its occurrences in step order, inserted once, sorted by pair and by context, and each query a few
+        searches (ng_online_occ_insert / _index / _query). The same counts as a fresh state advanced step by step,
+        without its launches and merges per step."""
+        taus, step_lo, step_hi = self._rule(rule, step_lo, step_hi)
+        cfg = self._check_config((), (1,), 0, count_levels)
+        tau, tau_in, last = taus if taus is not None else (self.tau, self.tau_in, self.max_step)
+        n, dev, lib = self.n, self.dev, self.lib
+        outs = self._device_outputs(cfg)
+        if rule == "segment":  # every position is a query
+            qpos, mq = None, n
+            rows = torch.arange(n, dtype=torch.int32, device=dev)
+        else:
+            order, steps = self._by_step([(tau_in, 0)], last + 1)[0]
+            qa, qb = self._range(steps, step_lo, step_hi)
+            rows = qpos = order[qa:qb]
+            mq = qb - qa
+        nc = len(count_levels)
+        bits = max(1, (last + 2).bit_length())
+        none = (1 << bits) - 1
+        cap = max(1 << 16, int(n / LOAD) + 1)
+        cbits = cap.bit_length()
+        u64s = [torch.empty(n, dtype=torch.int64, device=dev) for _ in range(4)]
+        u32s = [torch.empty(n, dtype=torch.int32, device=dev) for _ in range(4)]
+        ck = torch.empty(cap, dtype=torch.int64, device=dev)
+        bounds = torch.empty((cap, 2), dtype=torch.int32, device=dev)
+        first = torch.empty(n, dtype=torch.uint8, device=dev)
+        pre = torch.empty(n + 1, dtype=torch.int32, device=dev)
+        flags = torch.zeros((len(set(count_levels)), 2), dtype=torch.int32, device=dev)
+        ks = sorted(set(count_levels))
+        for k, flag in zip(ks, flags):
+            (key, ka, kb, akey), (val, va, vb, occ) = u64s, u32s
+            lib("ng_online_order", tau, n, self.bounds_dev, len(self.bounds) - 1, i32(k), u64(none), key, val)
+            lib.cub("sort_pairs", key, akey, val, occ, n, i32(0), i32(bits))
+            lib.fill(ck, -1)
+            lib("ng_online_occ_insert", self.tok, occ, akey, u64(none), n, i32(k), ck, u64(cap), i32(cbits), key, val,
+                flag)
+            lib.cub("sort_pairs", key, ka, val, va, n, i32(0), i32(16 + cbits))
+            lib.cub("sort_pairs", key, kb, val, vb, n, i32(16), i32(16 + cbits))
+            lib.cub("ng_online_occ_index", ka, va, kb, vb, n, i32(cbits), first, pre, bounds)
+            lib("ng_online_occ_query", self.tok, self.avail, self.has_next, qpos, mq, tau_in, akey, n, i32(k), ck,
+                u64(cap), bounds, vb, pre, ka, va, outs["tot"], outs["dist"], outs["cnt"], i32(nc),
+                i32(count_levels.index(k)))
+        for k, f in zip(ks, flags[:, 0].cpu().tolist()):
+            if f:
+                raise RuntimeError(f"k={k}: a table of the online state overflowed")
+        return outs, rows
+
+    def _range_rows(self, levels, buckets, entries, count_levels, step_lo, step_hi, rule, slots: int = 1,
+                    with_level: bool = False):
+        """A fresh state advanced over steps [0, step_hi), the queries of [step_lo, step_hi) answered. The rule
+        "segment" (online.rs:14-17: every position a query at its segment's start, an occurrence counted iff its next
+        token lies before that start) is the step rule with one step per segment in stream order: tau = tau_in = the
+        position's segment index makes an occurrence's alpha 1 + the segment of its next token, so it counts for a
+        query exactly when that segment lies before the query's; every step then runs as advance()'s do."""
+        taus, step_lo, step_hi = self._rule(rule, step_lo, step_hi)
         cfg = self._check_config(levels, buckets, entries, count_levels)
         st = self._new_state(cfg, taus)
         outs = self._device_outputs(cfg, slots, with_level)
@@ -463,7 +517,7 @@ class OnlineRows:
     def segment_counts(self, levels):
         """Every position's count rows under the rule "segment" (train_counts.rs's): tot uint32, dist uint16, cnt
         uint32 [n, len(levels)]."""
-        st, outs, _ = self._range_rows((), (1,), 0, levels, 0, 0, "segment")
+        outs, _ = self._range_counts(list(levels), 0, 0, "segment")
         return (outs["tot"].cpu().numpy().view(np.uint32), outs["dist"].cpu().numpy().view(np.uint16),
                 outs["cnt"].cpu().numpy().view(np.uint32))
 
@@ -486,5 +540,5 @@ class OnlineRows:
             raise ValueError(f"levels must be >= 1: {levels}")
         if tot.shape != (self.n, nl) or dist.shape != (self.n, nl) or cnt.shape != (self.n, nl):
             raise ValueError(f"outputs must be [{self.n}, {nl}]")
-        st, outs, rows = self._range_rows((), (1,), 0, levels, step_lo, step_hi, rule)
+        outs, rows = self._range_counts(list(levels), step_lo, step_hi, rule)
         self._copy_rows(outs, rows, None, None, None, tot, dist, cnt)

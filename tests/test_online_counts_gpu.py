@@ -1,0 +1,32 @@
+"""GPU: the count rows of a range of steps answered all at once (OnlineRows.counts: searches over each context's
+occurrences in step order) against the same range advanced step by step on the incremental state: overlapping and
+out-of-order spans, parts, steps without queries, ranges that start late or are empty, contexts longer than the stream,
+a hot context, both rules."""
+
+import numpy as np
+import pytest
+import torch
+
+from ngram_amd.online import OnlineRows
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,parts,vocab", [(1, 1, 3), (2, 1, 1), (40, 3, 2), (257, 1, 1), (6000, 5, 20), (6000, 2, 3)])
+@pytest.mark.parametrize("rule,lo,hi", [("step", 0, 12), ("step", 3, 5), ("step", 4, 4), ("segment", 0, 0)])
+def test_counts_match_the_stepwise_state(gpu, n, parts, vocab, rule, lo, hi):
+    rng = np.random.default_rng(n * 5 + parts)
+    tok = rng.integers(0, vocab, n).astype(np.uint16)
+    tok[rng.random(n) < 0.02] = 50256
+    bounds = [0, *sorted(rng.choice(np.arange(1, n), parts - 1, replace=False).tolist()), n] if parts > 1 else [0, n]
+    a = rng.integers(0, n + 1, 6 * parts)
+    b = np.minimum(a + rng.integers(0, max(2, n // 3), 6 * parts), n)
+    rows = OnlineRows(tok, bounds, np.stack([a, b, rng.integers(0, 10, 6 * parts)], 1))
+    levels = [3, 1, 2, 6, 60, 2]  # in any order, one of them twice
+    _, want, at = rows._range_rows((), (1,), 0, levels, lo, hi, rule)
+    got, at2 = rows._range_counts(levels, lo, hi, rule)
+    assert torch.equal(torch.sort(at).values, torch.sort(at2).values)
+    for name in ("tot", "dist", "cnt"):
+        assert torch.equal(got[name], want[name]), name
+    if n >= 6000 and (lo, hi) in ((0, 12), (0, 0)):  # the streams' draws leave counted contexts to compare
+        assert int(got["tot"].max()) > 3
