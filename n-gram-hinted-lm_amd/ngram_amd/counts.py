@@ -172,9 +172,10 @@ class CountBuild:
         n = cells.numel()
         rows = torch.empty(n + 2 * capacity, dtype=torch.int32, device=cells.device)
         work = torch.empty(self.lib.size("ng_batch_rows_work", n), dtype=torch.int32, device=cells.device)
-        total = torch.zeros(1, dtype=torch.int64, device=cells.device)
+        total = torch.empty(1, dtype=torch.int64, pin_memory=True)  # the kernel writes it where the host reads it
         self.lib("ng_batch_rows", cells, entries, n, capacity, rows, work, total)
-        m = int(total.item())
+        torch.cuda.current_stream().synchronize()
+        m = int(total[0])
         if m > capacity:
             raise AssertionError(f"{m} candidates overflow the rows' {capacity} entries")
         return rows

@@ -16,6 +16,9 @@ import torch
 from .build import lib_path
 
 _loaded: dict[str, ctypes.CDLL] = {}
+_ptr, _i64, _i32, _u64 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_uint64
+_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # None: a torch without a GPU backend
+_device = getattr(torch._C, "_cuda_getDevice", None)
 
 
 def load(path: str | Path | None = None) -> ctypes.CDLL:
@@ -54,19 +57,26 @@ class Lib:
     def __call__(self, name: str, *args) -> int:
         # the host side of every launch: kept short, since a build issues a few hundred of them back to back
         conv = []
+        put = conv.append
         for a in args:
-            if isinstance(a, torch.Tensor):
-                conv.append(ctypes.c_void_p(a.data_ptr()))
-            elif a is None:
-                conv.append(None)
+            t = type(a)
+            if t is torch.Tensor:
+                put(_ptr(a.data_ptr()))
+            elif t is int:
+                put(_i64(a))
+            elif a is None or t is _i32 or t is _u64:
+                put(a)
+            elif isinstance(a, torch.Tensor):
+                put(_ptr(a.data_ptr()))
             elif isinstance(a, int):
-                conv.append(ctypes.c_int64(a))
+                put(_i64(a))
             elif isinstance(a, (ctypes._SimpleCData, ctypes.Array)):
-                conv.append(a)
+                put(a)
             else:
                 raise TypeError(f"{name}: argument {a!r}")
-        conv.append(ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())))
-        rc = self._fn(name)(*conv)
+        put(_ptr(_stream(_device())))
+        fn = self._fns.get(name)
+        rc = (fn or self._fn(name))(*conv)
         if rc != 0:
             raise RuntimeError(f"{name} returned {rc}")
         return rc
