@@ -15,6 +15,7 @@ themselves is id-independent and equals the reference's. `memory` bounds the CPU
 
 from __future__ import annotations
 
+import functools
 import os
 
 import numpy as np
@@ -272,6 +273,12 @@ def train_counts(files, levels):
     return OnlineRows(tokens, bounds, np.zeros((0, 3), np.int64)).segment_counts(levels)
 
 
+@functools.lru_cache(maxsize=1)
+def _lib() -> Lib:
+    """The library's handle, looked up once: a call of a few tens of microseconds pays for it otherwise."""
+    return Lib()
+
+
 def features(counts: torch.Tensor, nb: int = 25):
     """The count mixture's features (record_367_gpu_counts/track_1_short/counts/mix.py features :22-31) of
     counts int32 [3, L, n] on the GPU: tot, dist, min(cnt, tot) (float32 [n, L]), the bin parameter index
@@ -287,5 +294,5 @@ def features(counts: torch.Tensor, nb: int = 25):
     cnt = torch.empty_like(tot)
     b = torch.empty((n, L), dtype=torch.int64, device=dev)
     s = torch.empty_like(b)
-    Lib()("ng_features", counts, i32(L), n, i32(nb), tot, dist, cnt, b, s)
+    _lib()("ng_features", counts, i32(L), n, i32(nb), tot, dist, cnt, b, s)
     return tot, dist, cnt, b, s
