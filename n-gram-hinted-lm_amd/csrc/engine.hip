@@ -960,10 +960,11 @@ static inline bool emit_mode_ok(int wbits, int dbits, int& mbits) {
 // positions set in bm): the positions whose context's bit is set in `final` emit their events as ng_scan_emit's
 // (regions, ev_count, dhist; region >= ng_emit_region(L, grid)), in its modes: wbits 0: mix64(pair key) with a
 // histogram of the top 8 bits; wbits in [17, 63]: kmix(pair key, wbits, mbits) (context ids below 2^(wbits - 16);
-// part.h; mbits 0: wbits) with a histogram of the top dbits bits (1 <= dbits <= 10), the 32-bit count's events.
+// part.h; mbits 0: wbits) with a histogram of the top dbits bits (1 <= dbits <= 10), the 32-bit count's events. key_add:
+// added to each pair key first (a context-id offset << 16: several levels counted in one id space).
 extern "C" int ng_scan_ids_emit(const u16* tok, i64 L, const u32* bm, const u32* ids, const u32* final, u64* ev,
                                 u64 region, u32* ev_count, u32* flags, int grid, u32* dhist, i64 dstride, int wbits,
-                                int dbits, int mbits, void* stream) {
+                                int dbits, int mbits, u64 key_add, void* stream) {
     if (grid <= 0 || region == 0 || region > 0xFFFFFFFFull || (dhist && dstride < grid)) return -1;
     if (!emit_mode_ok(wbits, dbits, mbits)) return -1;
     if ((L & 31) || ((uintptr_t)tok & 7) || ((uintptr_t)ids & 15)) return -1;  // the kernel's vector loads
@@ -975,7 +976,7 @@ extern "C" int ng_scan_ids_emit(const u16* tok, i64 L, const u32* bm, const u32*
             for (int d = 0; d < nd; ++d) fill_u32_n(dhist + (i64)d * dstride, 0u, grid, st);
         return (int)hipGetLastError();
     }
-    const EmitSink sk{ev, region, ev_count, 0, nullptr, dhist, dstride, 0, wbits, dbits, mbits};
+    const EmitSink sk{ev, region, ev_count, 0, nullptr, dhist, dstride, key_add, wbits, dbits, mbits};
     scan_ids_k<<<grid, 256, 0, st>>>(tok, L, bm, ids, final, sk, flags);
     return (int)hipGetLastError();
 }
@@ -1037,22 +1038,6 @@ extern "C" int ng_scan_emit_list(const u16* tok, const u64* plist, const u64* n_
     hipStream_t st = (hipStream_t)stream;
     LEVEL_DISPATCH(k, (scan_list_k<K, EmitSink><<<grid, 256, 0, st>>>(tok, plist, 0, k, vt, vcap, vrep, x, sk, flags, n_dev,
                                                                      bm_out)));
-    return (int)hipGetLastError();
-}
-
-// The list scan of ng_scan_sink over the first *n_dev entries of plist (n_max >= *n_dev; a device-side count, so no
-// host sync): hit bits and events (positions, what 1, or mixed pair keys, what 0) as ng_scan_sink's;
-// region >= ceil(n_max / (grid * 256)) * 256.
-extern "C" int ng_scan_list_dev(const u16* tok, int k, const u64* plist, const u64* n_dev, i64 n_max, const u64* vt,
-                                u64 vcap, const u32* vrep, const u16* x, u32* hit, int what, u64* ev, u64 region,
-                                u32* ev_count, u32* flags, int grid, u64 key_add, void* stream) {
-    if (grid <= 0 || !n_dev || !ev || (what != 0 && what != 1) || region == 0 || region > 0xFFFFFFFFull ||
-        (u64)n_max > (u64)grid * region)
-        return -1;
-    const EmitSink sk{ev, region, ev_count, what, hit, nullptr, 0, key_add};
-    hipStream_t st = (hipStream_t)stream;
-    LEVEL_DISPATCH(k, (scan_list_k<K, EmitSink><<<grid, 256, 0, st>>>(tok, plist, n_max, k, vt, vcap, vrep, x, sk, flags,
-                                                                     n_dev, nullptr)));
     return (int)hipGetLastError();
 }
 
@@ -1538,11 +1523,9 @@ extern "C" int ng_query_index(const u16* x, const int* avail, const int* pos, i6
 
 namespace {
 // One step of the longest match's active list: entry i (i < *n_dev) of act whose context (ctx_of[i]) has its hit bit
-// set matched level k (length[act[i]] = k); those with avail >= k + 1 go on to act_out. SPLIT: the entries that did
-// not match go on instead (the matched ones are done at length k). Each thread takes 4 entries; a block counts its
-// kept entries and matches and takes its place in act_out with one atomic each (a counter bumped per entry or per
-// wave would serialize).
-template <bool SPLIT>
+// set matched level k (length[act[i]] = k); those with avail >= k + 1 go on to act_out. Each thread takes 4 entries; a
+// block counts its kept entries and matches and takes its place in act_out with one atomic each (a counter bumped per
+// entry or per wave would serialize).
 __global__ void __launch_bounds__(256) act_next_k(const int* __restrict__ act, const u64* __restrict__ n_dev,
                                                   const int* __restrict__ ctx_of, const u32* __restrict__ hit,
                                                   const int* __restrict__ avail, int k, int* __restrict__ length,
@@ -1566,9 +1549,7 @@ __global__ void __launch_bounds__(256) act_next_k(const int* __restrict__ act, c
             if (c >= 0 && ((hit[c >> 5] >> (c & 31)) & 1u)) {
                 length[a[q]] = k;
                 ++nm;
-                keep[q] = !SPLIT && avail[a[q]] >= k + 1;
-            } else {
-                keep[q] = SPLIT;
+                keep[q] = avail[a[q]] >= k + 1;
             }
         }
         nk += keep[q];
@@ -1605,23 +1586,6 @@ __global__ void __launch_bounds__(256) act_next_k(const int* __restrict__ act, c
 }
 }  // namespace
 
-// The query index of the positions pos[0..*n_dev) (n_max >= *n_dev sizes the grid), compact ctx_of, without a host
-// sync: the table (cap + tail = slots) is EMPTY-filled here; counters[1] (a table too small) and
-// counters[2] (hashed keys that collided, k > 4) are added to, as ng_query_index's; the contexts are not counted.
-extern "C" int ng_query_index_dev(const u16* x, const int* avail, const int* pos, const u64* n_dev, i64 n_max, int k,
-                                  u64* table, u64 cap, u64 slots, u32* rep, int* ctx_of, u64* counters,
-                                  void* stream) {
-    if (cap == 0 || slots <= cap || slots > (1ull << 31) || !n_dev || !pos || n_max < 0) return -1;
-    hipStream_t st = (hipStream_t)stream;
-    fill_u32_n((u32*)table, 0xFFFFFFFFu, (i64)(2 * slots), st);
-    if (n_max == 0) return (int)hipGetLastError();
-    LEVEL_DISPATCH(k, (qindex_insert_k<K><<<grid_for(n_max, 256), 256, 0, st>>>(x, avail, pos, n_max, k, table, cap, slots,
-                                                                                rep, ctx_of, 1, counters, n_dev)));
-    if (k > 4)
-        qindex_verify_k<<<grid_for(n_max, 256), 256, 0, st>>>(x, pos, n_max, k, ctx_of, 1, rep, counters + 2, n_dev);
-    return (int)hipGetLastError();
-}
-
 // The longest match's active list, one level on: see act_next_k. n_out and matched are added to (zero them first);
 // act_out holds at least *n_dev entries; n_max >= *n_dev sizes the grid.
 extern "C" int ng_act_next(const int* act, const u64* n_dev, i64 n_max, const int* ctx_of, const u32* hit,
@@ -1629,18 +1593,501 @@ extern "C" int ng_act_next(const int* act, const u64* n_dev, i64 n_max, const in
                            void* stream) {
     if (!n_dev || n_max < 0) return -1;
     if (n_max > 0)
-        act_next_k<false><<<(int)((n_max + 1023) / 1024), 256, 0, (hipStream_t)stream>>>(
+        act_next_k<<<(int)((n_max + 1023) / 1024), 256, 0, (hipStream_t)stream>>>(
             act, n_dev, ctx_of, hit, avail, k, length, act_out, n_out, matched);
     return (int)hipGetLastError();
 }
 
-// The longest match's active list split at level k (see act_next_k): entries whose context's hit bit is set get
-// length k and are done; the others go to act_out. n_out and matched are added to (zero them first).
-extern "C" int ng_act_split(const int* act, const u64* n_dev, i64 n_max, const int* ctx_of, const u32* hit, int k,
-                            int* length, int* act_out, u64* n_out, u64* matched, void* stream) {
-    if (!n_dev || n_max < 0) return -1;
-    if (n_max > 0)
-        act_next_k<true><<<(int)((n_max + 1023) / 1024), 256, 0, (hipStream_t)stream>>>(
-            act, n_dev, ctx_of, hit, nullptr, k, length, act_out, n_out, matched);
+// ---------------------------------------------------------------------------------------------------------------
+// The longest match's host loop in few launches (ngram_amd/longest.py). Its levels are short: a level's launches and
+// the host work between them, not the work, bound all but the first few, so each step of the loop is one kernel and the
+// deep levels are launched from one call. A context's occurrence is marked with its level's number (lvl[id] = k), so
+// nothing is cleared between levels, and the query table is emptied slot by slot by the positions that filled it.
+// Measured (4M tokens, 256K positions, cap 32): 1278 launches and 11.7 ms a call with the levels' lists kept by framework
+// kernels and each list level indexed, scanned and packed by its own launches, 192 launches and 2.58 ms here.
+// ---------------------------------------------------------------------------------------------------------------
+
+namespace {
+
+// The block's `mine` kept entries of each thread (4 at most) placed: the block's base (one atomic on *n_out) + the entries
+// of earlier threads. Every thread of a 256-thread block calls it.
+__device__ __forceinline__ u64 place_in_block(u32 mine, u64* n_out, u32* s_wave, u64* s_base) {
+    const int lane = lane_id(), w = threadIdx.x / WAVE;
+    u32 incl = mine;
+#pragma unroll
+    for (int d = 1; d < WAVE; d <<= 1) {
+        const u32 o = (u32)__shfl_up((int)incl, d, WAVE);
+        if (lane >= d) incl += o;
+    }
+    __syncthreads();  // a previous call's values are read
+    if (lane == WAVE - 1) s_wave[w] = incl;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const u32 total = s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+        *s_base = total ? atomicAdd((unsigned long long*)n_out, (unsigned long long)total) : 0;
+    }
+    __syncthreads();
+    u64 at = *s_base + incl - mine;
+    for (int v = 0; v < w; ++v) at += s_wave[v];
+    return at;
+}
+
+// The queried positions (avail >= 1, and mask[i] where there is one) listed, a block's `chunk` in order, and counted by
+// min(avail, cap) (hist, cap + 1 entries). A block counts its chunk, takes its place with one atomic and reads the chunk
+// again to write it (same-address atomics serialize: one per 1024 positions of 64M would take 0.8 ms).
+__global__ void __launch_bounds__(256) lm_select_k(const int* __restrict__ avail, const unsigned char* __restrict__ mask,
+                                                   i64 n, i64 chunk, int cap, int* __restrict__ act, u64* n_act,
+                                                   u64* __restrict__ hist) {
+    __shared__ u32 s_wave[4], s_hist[MAXK + 1];
+    __shared__ u64 s_base;
+    const int lane = lane_id(), w = threadIdx.x / WAVE;
+    for (int h = threadIdx.x; h <= cap; h += 256) s_hist[h] = 0;
+    __syncthreads();
+    const i64 lo = (i64)blockIdx.x * chunk, hi = lo + chunk < n ? lo + chunk : n;
+    u32 mine = 0;
+    for (i64 i = lo + threadIdx.x; i < hi; i += 256) {
+        const int a = !mask || mask[i] ? avail[i] : 0;
+        if (a >= 1) {
+            ++mine;
+            atomicAdd(&s_hist[a < cap ? a : cap], 1u);
+        }
+    }
+    place_in_block(mine, n_act, s_wave, &s_base);  // the block's place; its entries then go in order of position
+    u64 at = s_base;
+    for (i64 r = lo; r < hi; r += 256) {
+        const i64 i = r + threadIdx.x;
+        const bool keep = i < hi && (!mask || mask[i]) && avail[i] >= 1;
+        const u64 b = __ballot(keep);
+        __syncthreads();  // the previous round's counts are read
+        if (lane == 0) s_wave[w] = (u32)__popcll(b);
+        __syncthreads();
+        u64 to = at + (u64)__popcll(b & lanemask_lt());
+        for (int v = 0; v < w; ++v) to += s_wave[v];
+        if (keep) act[to] = (int)i;
+        at += s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+    }
+    for (int h = threadIdx.x; h <= cap; h += 256)
+        if (s_hist[h]) atomicAdd((unsigned long long*)&hist[h], (unsigned long long)s_hist[h]);
+}
+
+// Level 1's index: each listed position's token is its context id, its bit set in member (2048 words, zeroed).
+__global__ void __launch_bounds__(256) lm_tok1_k(const u16* __restrict__ x, const int* __restrict__ act,
+                                                 const u64* __restrict__ n_dev, int* __restrict__ ctx_of,
+                                                 u32* __restrict__ member) {
+    __shared__ u32 s_mem[2048];
+    const i64 n = (i64)*n_dev;
+    for (int i = threadIdx.x; i < 2048; i += 256) s_mem[i] = 0;
+    __syncthreads();
+    for (i64 j = blockIdx.x * (i64)256 + threadIdx.x; j < n; j += (i64)gridDim.x * 256) {
+        const u32 t = x[act[j]];
+        ctx_of[j] = (int)t;
+        const u32 m = 1u << (t & 31);
+        if (!(s_mem[t >> 5] & m)) atomicOr(&s_mem[t >> 5], m);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 2048; i += 256)
+        if (s_mem[i]) atomicOr(&member[i], s_mem[i]);
+}
+
+// A deep level's scan: the listed corpus positions whose k-context is in the table, appended to hl in no order, their
+// contexts marked lvl[id] = k. A block gathers its hits in LDS and takes their place with one atomic when LM_STAGE - 1024
+// of them are there or its entries end.
+#define LM_STAGE 4096
+template <int K>
+__global__ void __launch_bounds__(256) lm_scan_k(const u16* __restrict__ tok, const u64* __restrict__ cand,
+                                                 const u64* __restrict__ n_dev, i64 n_max, int k,
+                                                 const u64* __restrict__ vt, u64 vcap, const u32* __restrict__ vrep,
+                                                 const u16* __restrict__ x, unsigned char* lvl, u64* __restrict__ hl,
+                                                 u64* n_hits, u32* flags) {
+    __shared__ u64 s_hit[LM_STAGE];
+    __shared__ u64 s_base;
+    __shared__ u32 s_n;
+    const i64 n = n_dev && (i64)*n_dev < n_max ? (i64)*n_dev : n_max;
+    const i64 stride = (i64)gridDim.x * 1024;
+    if (threadIdx.x == 0) s_n = 0;
+    for (i64 c0 = (i64)blockIdx.x * 1024; c0 < n; c0 += stride) {  // block-uniform
+        Walk2 wk[4];
+        u64 p[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const i64 j = c0 + q * 256 + threadIdx.x;
+            wk[q].key = EMPTY;
+            p[q] = 0;
+            if (j < n) {
+                p[q] = cand[j];
+                walk_begin2<K>(tok, (i64)p[q], k, vt, vcap, wk[q]);
+            }
+        }
+        __syncthreads();  // the stage is empty or holds the rounds before
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const u64 key = walk_end2<K>(tok, (i64)p[q], k, vt, vrep, x, flags, wk[q]);
+            const bool hit = key != EMPTY;
+            const u64 b = __ballot(hit);
+            if (!b) continue;  // wave-uniform
+            if (hit && lvl[key >> 16] != (unsigned char)k) lvl[key >> 16] = (unsigned char)k;
+            u32 at = 0;
+            if (lane_id() == 0) at = atomicAdd(&s_n, (u32)__popcll(b));
+            at = (u32)__shfl((int)at, 0, WAVE);
+            if (hit) s_hit[at + (u32)__popcll(b & lanemask_lt())] = p[q];
+        }
+        __syncthreads();
+        const u32 m = s_n;  // block-uniform
+        if (m > LM_STAGE - 1024 || c0 + stride >= n) {
+            if (threadIdx.x == 0) {
+                s_base = m ? atomicAdd((unsigned long long*)n_hits, (unsigned long long)m) : 0;
+                s_n = 0;
+            }
+            __syncthreads();
+            for (u32 i = threadIdx.x; i < m; i += 256) hl[s_base + i] = s_hit[i];
+        }
+    }
+}
+
+// After a deep level's scan: an active position whose context occurred (lvl[id] = k) matched it, length[i] = k; those
+// with avail >= k + 1 stay active (SPLIT: the ones that did not match do). Hashed contexts (k > 4) are checked against
+// their representative; the table's slots are emptied for the next level.
+template <bool SPLIT>
+__global__ void __launch_bounds__(256) lm_next_k(const u16* __restrict__ x, const int* __restrict__ avail,
+                                                 const int* __restrict__ act, const u64* __restrict__ n_dev, i64 n_max,
+                                                 const int* __restrict__ ctx_of, const unsigned char* __restrict__ lvl,
+                                                 const u32* __restrict__ rep, int k, u64* __restrict__ table,
+                                                 int* __restrict__ length, int* __restrict__ act_out, u64* n_out,
+                                                 u64* matched, u64* bad) {
+    __shared__ u32 s_wave[4], s_match;
+    __shared__ u64 s_base;
+    const i64 n = n_dev && (i64)*n_dev < n_max ? (i64)*n_dev : n_max;
+    const i64 b0 = (i64)blockIdx.x * 1024 + threadIdx.x * 4;
+    if ((i64)blockIdx.x * 1024 >= n) return;  // block-uniform
+    if (threadIdx.x == 0) s_match = 0;
+    int a[4];
+    bool keep[4];
+    u32 mine = 0, nm = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const i64 i = b0 + q;
+        keep[q] = false;
+        a[q] = 0;
+        if (i < n) {
+            a[q] = act[i];
+            const int c = ctx_of[i];
+            bool m = false;
+            if (c >= 0) {
+                m = lvl[c] == (unsigned char)k;
+                if (k > 4 && !same_tokens_rt(x + a[q] + 1, x + (i64)rep[c] + 1, k))
+                    atomicAdd((unsigned long long*)bad, 1ull);
+                table[c] = EMPTY;
+            }
+            if (m) {
+                length[a[q]] = k;
+                ++nm;
+            }
+            keep[q] = SPLIT ? !m : m && avail[a[q]] >= k + 1;
+            mine += keep[q];
+        }
+    }
+    u64 at = place_in_block(mine, n_out, s_wave, &s_base);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        if (keep[q]) act_out[at++] = a[q];
+#pragma unroll
+    for (int d = WAVE / 2; d > 0; d >>= 1) nm += (u32)__shfl_down((int)nm, d, WAVE);
+    if (lane_id() == 0 && nm) atomicAdd(&s_match, nm);
+    __syncthreads();
+    if (threadIdx.x == 0 && s_match) atomicAdd((unsigned long long*)matched, (unsigned long long)s_match);
+}
+
+// The active positions of a bitmap level whose match ends there (length k): their group context id (base + ctx_of) and its
+// bit in `final` (the level's bits).
+__global__ void __launch_bounds__(256) lm_final_k(const int* __restrict__ act, i64 n, const int* __restrict__ ctx_of,
+                                                  const int* __restrict__ length, int k, int base,
+                                                  int* __restrict__ fid, u32* final) {
+    const i64 j = blockIdx.x * (i64)256 + threadIdx.x;
+    if (j >= n) return;
+    const int i = act[j], c = ctx_of[j];
+    if (length[i] != k || c < 0) return;
+    fid[i] = base + c;
+    const u32 m = 1u << (c & 31);
+    if (!(final[c >> 5] & m)) atomicOr(&final[c >> 5], m);
+}
+
+// The key of a k-context among contexts of several lengths.
+__device__ __forceinline__ u64 mixed_key(u64 h, int k) { return key_finish(h ^ ((u64)k * 0xA24BAED4963EE407ull)); }
+
+// The list levels' final contexts in one table: each active position of length k >= k0 inserts its k-context.
+// counters[3 k + 1]: as ng_query_index's counters[1], for that level.
+__global__ void __launch_bounds__(256) lm_mixed_insert_k(const u16* __restrict__ x, const int* __restrict__ act, i64 n,
+                                                         const int* __restrict__ length, int k0, u64* table, u64 cap,
+                                                         u64 slots, u32* __restrict__ rep, int base,
+                                                         int* __restrict__ fid, u64* counters) {
+    const i64 j = blockIdx.x * (i64)256 + threadIdx.x;
+    if (j >= n) return;
+    const i64 i = act[j];
+    const int k = length[i];
+    if (k < k0) return;
+    bool gap = false;
+    const u64 key = mixed_key(ctx_hash_rt(x + i + 1, k, gap), k);
+    u64 s = __umul64hi(key, cap);
+    i64 slot = -1;
+    for (int walked = 0;; ++walked, ++s) {
+        if (s + 1 >= slots || walked == QI_MAXWALK) {  // the last slot must stay empty; a table far too small
+            atomicOr((unsigned int*)&counters[3 * k + 1], s + 1 >= slots ? 1u : 2u);
+            break;
+        }
+        u64 cur = table[s];
+        if (cur == EMPTY) {
+            cur = atomicCAS((unsigned long long*)&table[s], EMPTY, key);
+            if (cur == EMPTY) {
+                rep[s] = (u32)i;
+                cur = key;
+            }
+        }
+        if (cur == key) {
+            slot = (i64)s;
+            break;
+        }
+    }
+    fid[i] = slot >= 0 ? base + (int)slot : -1;
+}
+
+// Each inserted position's context against its slot's representative: another length or other tokens share a key.
+__global__ void __launch_bounds__(256) lm_mixed_verify_k(const u16* __restrict__ x, const int* __restrict__ act, i64 n,
+                                                         const int* __restrict__ length, int k0,
+                                                         const u32* __restrict__ rep, int base,
+                                                         const int* __restrict__ fid, u64* counters) {
+    const i64 j = blockIdx.x * (i64)256 + threadIdx.x;
+    if (j >= n) return;
+    const i64 i = act[j];
+    const int k = length[i];
+    if (k < k0 || fid[i] < 0) return;
+    const i64 r = rep[fid[i] - base];
+    if (length[r] != k || !same_tokens_rt(x + i + 1, x + r + 1, k))
+        atomicAdd((unsigned long long*)&counters[3 * k + 2], 1ull);
+}
+
+// The list levels' hit lists laid end to end: list t holds level k[t]'s corpus positions at p[t], from off[t] on.
+struct LmLists {
+    const u64* p[MAXK];
+    i64 off[MAXK + 1];
+    int k[MAXK];
+    int n;
+};
+
+// Every list level's positions probed for their own level's final contexts; hits' events as an emitting scan's.
+__global__ void __launch_bounds__(256) lm_mixed_scan_k(const u16* __restrict__ tok, LmLists ls,
+                                                       const u64* __restrict__ vt, u64 vcap,
+                                                       const u32* __restrict__ rep, const u16* __restrict__ x,
+                                                       const int* __restrict__ length, EmitSink sink, u32* flags) {
+    __shared__ SinkShared ss;
+    __shared__ i64 s_off[MAXK + 1];
+    __shared__ const u64* s_p[MAXK];
+    __shared__ int s_k[MAXK];
+    for (int t = threadIdx.x; t < ls.n; t += 256) {
+        s_off[t] = ls.off[t];
+        s_p[t] = ls.p[t];
+        s_k[t] = ls.k[t];
+    }
+    sink_begin(sink, &ss);
+    __syncthreads();
+    const i64 total = ls.off[ls.n];
+    for (i64 e0 = (i64)blockIdx.x * 256; e0 < total; e0 += (i64)gridDim.x * 256) {
+        const i64 e = e0 + threadIdx.x;
+        u64 key = EMPTY;
+        i64 p = 0;
+        if (e < total) {
+            int t = 0, hi = ls.n;  // the last list with off <= e
+            while (hi - t > 1) {
+                const int m = (t + hi) >> 1;
+                if (s_off[m] <= e) t = m;
+                else hi = m;
+            }
+            const int k = s_k[t];
+            p = (i64)s_p[t][e - s_off[t]];
+            const u32 nxt = tok[p];
+            bool gap = p < k || nxt == SENT;
+            if (!gap) {
+                const u64 h = ctx_hash_rt(tok + p, k, gap);
+                if (!gap) {
+                    const u64 want = mixed_key(h, k);
+                    u64 s = __umul64hi(want, vcap);
+                    u64 cur = vt[s];
+                    while (cur != want && cur != EMPTY) cur = vt[++s];  // the table ends with an empty slot
+                    if (cur == want) {
+                        const i64 r = rep[s];
+                        if (length[r] == k && same_tokens_rt(tok + p, x + r + 1, k)) key = (s << 16) | nxt;
+                        else atomicAdd(&flags[1], 1u);
+                    }
+                }
+            }
+        }
+        const bool hit = key != EMPTY;
+        emit_wave(sink, &ss, __ballot(hit), hit, key, p, flags);
+    }
+    sink_end(sink, &ss);
+}
+
+// Positions of group ids below n_ids: their context's top entry (CtxRecord<1>), the id then dropped (fid[i] = -1).
+__global__ void __launch_bounds__(256) lm_top1_k(int* __restrict__ fid, i64 n, i64 n_ids, const u32* __restrict__ rec,
+                                                 const u32* __restrict__ dist, u16* __restrict__ nxt,
+                                                 u32* __restrict__ cnt) {
+    const i64 i = blockIdx.x * (i64)256 + threadIdx.x;
+    if (i >= n) return;
+    const int c = fid[i];
+    if (c < 0 || c >= n_ids) return;
+    fid[i] = -1;
+    if (!dist[c]) return;
+    const uint4 r = *(const uint4*)(rec + (i64)c * CtxRecord<1>::WORDS);
+    nxt[i] = (u16)r.z;
+    cnt[i] = r.w;
+}
+
+static int launch_lm_scan(const u16* tok, const u64* cand, const u64* n_dev, i64 n_max, int k, const u64* vt, u64 vcap,
+                          const u32* vrep, const u16* x, unsigned char* lvl, u64* hl, u64* n_hits, u32* flags, int grid,
+                          hipStream_t st) {
+    LEVEL_DISPATCH(k, (lm_scan_k<K><<<grid, 256, 0, st>>>(tok, cand, n_dev, n_max, k, vt, vcap, vrep, x, lvl, hl, n_hits,
+                                                         flags)));
+    return 0;
+}
+
+static int launch_lm_insert(const u16* x, const int* avail, const int* act, i64 n_max, int k, u64* table, u64 cap,
+                            u64 slots, u32* rep, int* ctx_of, u64* counters, const u64* n_dev, hipStream_t st) {
+    LEVEL_DISPATCH(k, (qindex_insert_k<K><<<grid_for(n_max, 256), 256, 0, st>>>(x, avail, act, n_max, k, table, cap, slots,
+                                                                                rep, ctx_of, 1, counters, n_dev)));
+    return 0;
+}
+}  // namespace
+
+// The longest match's queried positions: those with avail >= 1 (and mask[i] != 0; mask may be NULL) listed in act (room
+// for n), *n_act += their number, hist[min(avail, cap)] += 1 for each (cap + 1 u64; both zeroed by the caller).
+extern "C" int ng_lm_select(const int* avail, const unsigned char* mask, i64 n, int cap, int* act, u64* n_act, u64* hist,
+                            void* stream) {
+    if (n < 0 || cap < 1 || cap > MAXK || !n_act || !hist || (n && (!avail || !act))) return -1;
+    if (n) {
+        const i64 chunk = n <= 4096 * 2048ll ? 4096 : ((n + 2047) / 2048 + 255) / 256 * 256;
+        lm_select_k<<<(unsigned)((n + chunk - 1) / chunk), 256, 0, (hipStream_t)stream>>>(avail, mask, n, chunk, cap, act,
+                                                                                        n_act, hist);
+    }
+    return (int)hipGetLastError();
+}
+
+// Level 1's index over act[0..*n_dev) (at most n_max): ctx_of[j] = the position's token, member (2048 words, zeroed) its
+// bit, for ng_scan_tok1.
+extern "C" int ng_lm_tok1(const u16* x, const int* act, const u64* n_dev, i64 n_max, int* ctx_of, u32* member,
+                          void* stream) {
+    if (n_max < 0 || !n_dev || !member) return -1;
+    const int g = grid_for(n_max, 4096);
+    if (n_max) lm_tok1_k<<<g < 1024 ? g : 1024, 256, 0, (hipStream_t)stream>>>(x, act, n_dev, ctx_of, member);
+    return (int)hipGetLastError();
+}
+
+// The deep levels k0..cap of the existence phase from the active positions act0[0..n0) (avail >= k0) and the corpus
+// positions cand[0..nc0) that hit level k0 - 1, three launches a level. first: level cap is tried before the others, and
+// the positions matching it are done; the levels in between are then walked by the rest only.
+// table (cap_q < slots u64, EMPTY; left EMPTY), rep and lvl (a byte, zeroed) per slot, ctx_of, act_a and act_b (n0 each)
+// are scratch; hl holds (cap - k0 + 1) lists of nc0. meta (zeroed, u64 [cap - k0 + 2][6]), row k - k0: positions kept for
+// the next level, positions matched, corpus hits (the length of hl's list k - k0), then ng_query_index's counters; the
+// last row's first two: the positions going on from level cap's trial, and those matched there (its hits and counters
+// are level cap's row's).
+extern "C" int ng_lm_levels(const u16* tok, const u16* x, const int* avail, int k0, int cap, int first, const int* act0,
+                            i64 n0, int* act_a, int* act_b, const u64* cand, i64 nc0, u64* table, u64 cap_q, u64 slots,
+                            u32* rep, int* ctx_of, unsigned char* lvl, u64* hl, int* length, u64* meta, u32* flags,
+                            int grid, void* stream) {
+    if (k0 < 1 || cap < k0 || cap > MAXK || n0 < 1 || nc0 < 0 || cap_q == 0 || slots <= cap_q || slots > (1ull << 31) ||
+        grid <= 0 || !act0 || !act_a || !act_b || !table || !rep || !ctx_of || !lvl || !hl || !length || !meta || !flags)
+        return -1;
+    hipStream_t st = (hipStream_t)stream;
+    const int nlev = cap - k0 + 1, gn = (int)((n0 + 1023) / 1024);
+    const int gs = (int)((nc0 + 1023) / 1024 < grid ? (nc0 + 1023) / 1024 : grid);
+    const i64 room = nc0 > 0 ? nc0 : 1;
+    const int* cur = act0;
+    const u64* cur_n = nullptr;
+    const u64* from = cand;
+    const u64* from_n = nullptr;
+    auto level = [&](int k, u64* row, u64* out_n, u64* out_m, int* out, bool split) -> int {
+        int rc = launch_lm_insert(x, avail, cur, n0, k, table, cap_q, slots, rep, ctx_of, row + 3, cur_n, st);
+        if (rc) return rc;
+        if (gs > 0 && (rc = launch_lm_scan(tok, from, from_n, nc0, k, table, cap_q, rep, x, lvl, hl + (i64)(k - k0) * room,
+                                           row + 2, flags, gs, st)))
+            return rc;
+        if (split)
+            lm_next_k<true><<<gn, 256, 0, st>>>(x, avail, cur, cur_n, n0, ctx_of, lvl, rep, k, table, length, out, out_n,
+                                                out_m, row + 5);
+        else
+            lm_next_k<false><<<gn, 256, 0, st>>>(x, avail, cur, cur_n, n0, ctx_of, lvl, rep, k, table, length, out, out_n,
+                                                 out_m, row + 5);
+        return (int)hipGetLastError();
+    };
+    int rc = 0;
+    if (first) {
+        u64* last = meta + (i64)nlev * 6;
+        if ((rc = level(cap, meta + (i64)(nlev - 1) * 6, last, last + 1, act_a, true))) return rc;
+        cur = act_a;
+        cur_n = last;
+    }
+    for (int k = k0; k <= (first ? cap - 1 : cap); ++k) {
+        u64* row = meta + (i64)(k - k0) * 6;
+        int* out = cur == act_a ? act_b : act_a;
+        if ((rc = level(k, row, row, row + 1, out, false))) return rc;
+        cur = out;
+        cur_n = row;
+        from = hl + (i64)(k - k0) * room;
+        from_n = row + 2;
+    }
+    return rc;
+}
+
+// A bitmap level's final positions (those of act[0..n) with length k): fid[i] = base + ctx_of[j], and ctx_of[j]'s bit in
+// final (zeroed by the caller).
+extern "C" int ng_lm_final(const int* act, i64 n, const int* ctx_of, const int* length, int k, int base, int* fid,
+                           u32* final, void* stream) {
+    if (n < 0 || base < 0) return -1;
+    if (n) lm_final_k<<<grid_for(n, 256), 256, 0, (hipStream_t)stream>>>(act, n, ctx_of, length, k, base, fid, final);
+    return (int)hipGetLastError();
+}
+
+// The final contexts of the list levels, k0 and deeper, in one table (EMPTY-filled, cap_q < slots): each position of
+// act[0..n) of length k >= k0 inserts its k-context, fid[i] = base + its slot, rep its representative; counters (u64 [65][3],
+// zeroed): row k as ng_query_index's.
+extern "C" int ng_lm_index(const u16* x, const int* act, i64 n, const int* length, int k0, u64* table, u64 cap_q, u64 slots,
+                           u32* rep, int base, int* fid, u64* counters, void* stream) {
+    if (n < 0 || k0 < 1 || cap_q == 0 || slots <= cap_q || slots > (1ull << 31) || base < 0) return -1;
+    hipStream_t st = (hipStream_t)stream;
+    if (n) {
+        lm_mixed_insert_k<<<grid_for(n, 256), 256, 0, st>>>(x, act, n, length, k0, table, cap_q, slots, rep, base, fid,
+                                                            counters);
+        lm_mixed_verify_k<<<grid_for(n, 256), 256, 0, st>>>(x, act, n, length, k0, rep, base, fid, counters);
+    }
+    return (int)hipGetLastError();
+}
+
+// The corpus positions of nl (1..64) lists (lists[t * 3 ...] = device pointer (u64 positions), their number, level k; host
+// memory) probed for their level's contexts in ng_lm_index's table; hits' events as ng_scan_emit's in its W-bit mode, with
+// key_add. region >= ceil(total / (grid * 256)) * 256.
+extern "C" int ng_lm_lists_emit(const u16* tok, const i64* lists, int nl, const u64* vt, u64 vcap, const u32* rep,
+                                const u16* x, const int* length, u64* ev, u64 region, u32* ev_count, u32* flags, int grid,
+                                u32* dhist, i64 dstride, int wbits, int dbits, int mbits, u64 key_add, void* stream) {
+    if (grid <= 0 || nl < 1 || nl > MAXK || !lists || region == 0 || region > 0xFFFFFFFFull || (dhist && dstride < grid) ||
+        !wbits || !emit_mode_ok(wbits, dbits, mbits))
+        return -1;
+    LmLists ls{};
+    ls.n = nl;
+    for (int t = 0; t < nl; ++t) {
+        const i64* f = lists + 3 * (i64)t;
+        if (f[1] < 0 || f[2] < 1 || f[2] > MAXK || (f[1] && !f[0])) return -1;
+        ls.p[t] = (const u64*)f[0];
+        ls.k[t] = (int)f[2];
+        ls.off[t + 1] = ls.off[t] + f[1];
+    }
+    if ((u64)ls.off[nl] > (u64)grid * region) return -1;
+    const EmitSink sk{ev, region, ev_count, 0, nullptr, dhist, dstride, key_add, wbits, dbits, mbits};
+    lm_mixed_scan_k<<<grid, 256, 0, (hipStream_t)stream>>>(tok, ls, vt, vcap, rep, x, length, sk, flags);
+    return (int)hipGetLastError();
+}
+
+// Positions i < n with 0 <= fid[i] < n_ids: nxt / cnt = their context's top entry from its record (topk 1), where
+// dist[id] is not 0; fid[i] = -1 afterwards.
+extern "C" int ng_lm_top1(int* fid, i64 n, i64 n_ids, const u32* rec, const u32* dist, u16* nxt, u32* cnt, void* stream) {
+    if (n < 0 || n_ids < 0) return -1;
+    if (n) lm_top1_k<<<grid_for(n, 256), 256, 0, (hipStream_t)stream>>>(fid, n, n_ids, rec, dist, nxt, cnt);
     return (int)hipGetLastError();
 }

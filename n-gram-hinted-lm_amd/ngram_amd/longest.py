@@ -9,19 +9,21 @@ Two phases, both on libngram_amd.so. Existence, k = 1, 2, ...: the query context
 (a query index per level over the list of positions still matching), the corpus positions whose (k-1)-context
 matched (a hit bitmap while dense, then a position list) probed for their k-context (ng_scan_exist: a bitmap, a
 per-context hit bit and each hit position's context id, no counting), until no position matches; once the lists
-shrink slowly, the remaining levels run as one stream of launches with device-side counts (no host sync per level).
-A match is monotone in k (kgram.rs:12-15), so each position's length is its last matching level. Then counting,
-only for each position's final context: a bitmap level's hit positions whose stored context id is final emit their
-(context, next) events (ng_scan_ids_emit: no second query index or probe); a list level's final contexts get a query
-index and its listed positions are probed, the list levels counted together. The events are partitioned and counted
-in LDS (partcount.py: no global atomics, so the hot pairs of short contexts cost no serialized chains), each
-context's top entry made from its pairs (ng_ctx_summary) and gathered to its positions (ng_pos_summary).
+shrink slowly, the remaining levels run as one stream of launches with device-side counts (ng_lm_levels: no host sync
+per level). A match is monotone in k (kgram.rs:12-15), so each position's length is its last matching level. Then
+counting, only for each position's final context: a bitmap level's hit positions whose stored context id is final emit
+their (context, next) events (ng_scan_ids_emit: no second query index or probe); the list levels' final contexts share
+one table, their key holding their length, which their listed positions are probed against (ng_lm_index,
+ng_lm_lists_emit). The events of one level, or of a small corpus's levels together, are partitioned and counted in LDS
+(partcount.py: no global atomics, so the hot pairs of short contexts cost no serialized chains), each context's top
+entry made from its pairs and gathered to its positions (ng_lm_top1).
 
 Surfaces: `longest_match(...)` on GPU tensors, and `LongestMatch.create(files, tokens, threads, cpus)` /
 `build() -> dict` in cache_ladder's shape (cache_ladder/src/lib.rs:1-8, cache_ladder.pyi)."""
 
 from __future__ import annotations
 
+import ctypes
 import os
 import time
 from types import SimpleNamespace
@@ -36,12 +38,6 @@ from .lib import Lib, i32, u64
 from .partcount import (W_MAX, count32, count_events, emit_region, first_digit, key_mbits, pack_events, pbits32_max,
                         runs_fit, summarize, w_bits)
 from .qindex import LOAD as QLOAD, TAIL as QTAIL, QueryIndex
-
-
-def _popcount(lib: Lib, bm: torch.Tensor) -> int:
-    c = torch.zeros(1, dtype=torch.int64, device=bm.device)
-    lib("popcount", bm, bm.numel(), c)
-    return int(c.item())
 
 
 _RATIO: dict[int, float] = {}  # distinct pairs per counted event at each level, from the last count (sizes partitions)
@@ -66,20 +62,27 @@ def longest_match(tok: torch.Tensor, x: torch.Tensor, avail: torch.Tensor, cap: 
     dev = x.device
     N, L = x.numel(), tok.numel()
     nwords = L // 32
-    grid = torch.cuda.get_device_properties(dev).multi_processor_count * SCAN_BLOCKS_PER_CU
+    # scan blocks: as many as the device takes, but at least 8192 positions each (a block's hits are a segment of the
+    # count's first pass, whose cost per segment a small corpus would otherwise pay thousands of times)
+    grid = max(1, min(torch.cuda.get_device_properties(dev).multi_processor_count * SCAN_BLOCKS_PER_CU, -(-L // 8192)))
     t0 = time.perf_counter()
-    length = torch.zeros(N, dtype=torch.int32, device=dev)
-    # the queried positions, as a list; each level keeps the ones still matching (the lists shrink fast)
-    sel = avail >= 1 if query is None else (avail >= 1) & query
-    act = torch.nonzero(sel).squeeze(1).to(torch.int32)
-    # eligible at level k: queried positions with avail >= k (one histogram for every level)
-    elig = torch.bincount(avail[act.long()].clamp_max(cap).long(), minlength=cap + 1).flip(0).cumsum(0).flip(0)
-    elig = elig.cpu().tolist()
+    length = elib.zeros(N, torch.int32, dev)
+    # the queried positions, as a list; each level keeps the ones still matching (the lists shrink fast). meta holds what
+    # the host reads: the positions by min(avail, cap), then per level the positions kept for the next one, those matched,
+    # the corpus positions hit, and the query index's counters (row 0: the queried positions)
+    meta = elib.zeros(cap + 1 + 6 * (cap + 2), torch.int64, dev)
+    hist, rows = meta[: cap + 1], meta[cap + 1 :].view(cap + 2, 6)
+    act = torch.empty(max(N, 1), dtype=torch.int32, device=dev)
+    mask = None
+    if query is not None:
+        mask = query if query.dtype in (torch.bool, torch.uint8) else query.bool()
+        mask = mask.expand(N).contiguous().view(torch.uint8)
+    elib("ng_lm_select", avail, mask, N, i32(cap), act, rows[0], hist)
     # each level's hit set (the corpus positions whose k-context is a query context of the level): a bitmap while
     # dense, then, once sparse, a list of positions, which the next level scans instead of every bitmap word
-    levels: list[tuple[str, torch.Tensor, int]] = []
+    levels: list[tuple] = []
     ladder = []
-    flags = torch.zeros(2, dtype=torch.int32, device=dev)
+    flags = elib.zeros(2, torch.int32, dev)
     # the prefix rule for the bitmap scans (a device flag, no host sync): with every position queried, a position
     # still active at level k has its predecessor active at level k - 1 (its shorter context occurs wherever the
     # longer one does), so where avail is segment-shaped a level's context also has its prefix among the level before's
@@ -89,118 +92,91 @@ def longest_match(tok: torch.Tensor, x: torch.Tensor, avail: torch.Tensor, cap: 
     if query is None:
         pre = torch.empty(1, dtype=torch.int32, device=dev)
         elib("ng_avail_closed", avail, N, pre)
+    elig: list = []
+    deep = None  # the list levels' first level and its active positions
+    n_act = N  # level 1's is read with its results; later levels' are exact
     for k in range(1, cap + 1):
-        act = act[avail[act.long()] >= k]
-        if act.numel() == 0:
-            break
-        if levels and levels[-1][0] == "list" and DEVICE_LEVELS:
-            # the sparse levels' lists shrink slowly from here on: the remaining levels run without a host sync
-            for k2, hl, nh, matched in _exist_device(elib, tok, L, x, avail, act, k, cap, levels[-1][1], length,
-                                                    flags, grid):
-                levels.append(("list", hl, nh))
-                ladder.append((k2, int(elig[k2]), matched))
+        if n_act == 0:
             break
         prev = levels[-1] if levels else None
-        if prev is None and k == 1:
+        sparse = prev is not None and (prev[0] == "list" or prev[2] * LIST_DIV < L)
+        if sparse and deep is None:
+            deep = (k, act, n_act)
+        if sparse and DEVICE_LEVELS:
+            # the sparse levels' lists shrink slowly from here on: the remaining levels run without a host sync
+            cand = prev[1] if prev[0] == "list" else _bits_list(elib, prev[1], prev[2])
+            for k2, hl, nh, matched in _exist_device(elib, tok, L, x, avail, act[:n_act], k, cap, cand, length, flags,
+                                                     grid):
+                levels.append(("list", hl, nh))
+                ladder.append((k2, elig[k2], matched))
+            break
+        row = rows[k]
+        nxt_act = torch.empty(max(n_act, 1), dtype=torch.int32, device=dev)
+        if k == 1:
             # level 1: a 1-context's id is its token, so no query table (ng_scan_tok1 holds the query tokens' set)
-            vi = _tok1_index(x, act)
-            hit = torch.zeros(2048, dtype=torch.int32, device=dev)
+            ctx_of = torch.empty(max(N, 1), dtype=torch.int32, device=dev)
+            member = elib.zeros(2048, torch.int32, dev)
+            elib("ng_lm_tok1", x, act, rows[0], N, ctx_of, member)
+            hit = elib.zeros(2048, torch.int32, dev)
             bm = torch.empty(nwords, dtype=torch.int32, device=dev)
             # no stored ids: a hit's context id is the token before it, which the counting scan reads itself
-            elib("ng_scan_tok1", tok, L, vi.member, bm, hit, None, i32(TOK1_GRID))
-            levels.append(("bm", bm, _popcount(lib, bm), None, act, vi.ctx_of, vi.ids))
-            ctx = vi.ctx_of.long()
-            act = act[((hit[ctx >> 5] >> (ctx & 31)) & 1) != 0]
-            length[act.long()] = k
-            ladder.append((k, int(elig[k]), int(act.numel())))
-            del vi, hit, ctx
-            continue
-        per = _CONTEXTS.get(k)
-        vi = QueryIndex(elib, x, avail, k, act, compact=True,
-                        expect=None if per is None else int(per * act.numel()) + 1)
-        _CONTEXTS[k] = vi.n / max(1, act.numel())
-        hit = torch.zeros((vi.ids + 31) // 32, dtype=torch.int32, device=dev)  # a bit per context id
-        if prev is not None and (prev[0] == "list" or prev[2] * LIST_DIV < L):
-            cand = prev[1] if prev[0] == "list" else _bits_list(elib, prev[1], prev[2])
-            hl, nh = _scan_list(elib, tok, L, k, vi, x, cand, hit, 1, flags, grid)
-            levels.append(("list", hl, nh))
+            elib("ng_scan_tok1", tok, L, member, bm, hit, None, i32(TOK1_GRID))
+            level = ["bm", bm, 0, None, act, ctx_of, 65536]
+            lib("popcount", bm, nwords, row[2:])
+            elib("ng_act_next", act, rows[0], N, ctx_of, hit, avail, i32(1), length, nxt_act, row, row[1:])
+            host = meta.cpu().tolist()
+            n_act = host[cap + 1]
+            elig = [sum(host[j : cap + 1]) for j in range(cap + 1)]
+            if n_act == 0:
+                break
+        elif sparse:
+            host = _exist_list(elib, tok, L, x, avail, act, n_act, k, prev, length, flags, grid, row, nxt_act)
+            level = ["list", host.pop(), 0]
         else:
-            bm = torch.empty(nwords, dtype=torch.int32, device=dev)
-            ids = torch.empty(L, dtype=torch.int32, device=dev)  # each hit position's context id, for the counting
-            mode = 0 if prev is None or prev[2] * 2 > L else 2  # a lane per position while the gate is dense
-            elib("ng_scan_exist", tok, L, i32(k), None if prev is None else prev[1], bm, vi.table, u64(vi.cap),
-                 vi.rep, x, hit, ids, flags, i32(grid), i32(mode), pre)
-            levels.append(("bm", bm, _popcount(lib, bm), ids, act, vi.ctx_of, vi.ids))
-        ctx = vi.ctx_of.long()
-        c = ctx.clamp_min(0)
-        act = act[(ctx >= 0) & (((hit[c >> 5] >> (c & 31)) & 1) != 0)]
-        length[act.long()] = k
-        ladder.append((k, int(elig[k]), int(act.numel())))
-        del vi, hit, ctx
+            per = _CONTEXTS.get(k)
+            expect = None if per is None else int(per * n_act) + 1
+            for checked in (False, True):
+                # sized from the last call's contexts, its counters read with the level's results; an index that proves
+                # too small for this call's contexts is built again, sized and checked as it is built
+                vi = QueryIndex(elib, x, avail, k, act[:n_act], compact=True, expect=expect,
+                                defer=not checked and expect is not None, counters=row[3:6])
+                hit = elib.zeros((vi.ids + 31) // 32, torch.int32, dev)  # a bit per context id
+                bm = torch.empty(nwords, dtype=torch.int32, device=dev)
+                ids = torch.empty(L, dtype=torch.int32, device=dev)  # each hit position's context id, for the counting
+                mode = 0 if prev[2] * 2 > L else 2  # a lane per position while the gate is dense
+                elib("ng_scan_exist", tok, L, i32(k), prev[1], bm, vi.table, u64(vi.cap), vi.rep, x, hit, ids, flags,
+                     i32(grid), i32(mode), pre)
+                lib("popcount", bm, nwords, row[2:])
+                elib("ng_act_next", act, rows[k - 1] if k > 1 else rows[0], n_act, vi.ctx_of, hit, avail, i32(k), length,
+                     nxt_act, row, row[1:])
+                host = rows[k].cpu().tolist()
+                if vi.n is not None:
+                    break
+                if host[5]:
+                    raise RuntimeError(f"k={k}: {host[5]} query positions collide with another context's key")
+                vi.n = host[3]
+                if not host[4] and vi.n <= 2 * QLOAD * vi.cap:
+                    break
+                elib.fill(row, 0)
+            _CONTEXTS[k] = vi.n / max(1, n_act)
+            level = ["bm", bm, 0, ids, act, vi.ctx_of, vi.ids]
+            del vi, hit
+        r = host[-6:] if k > 1 else host[cap + 1 + 6 * k : cap + 1 + 6 * k + 6]
+        level[2] = r[2]
+        if level[0] == "bm":
+            level.append(n_act)
+        else:
+            level[1] = level[1][: r[2]]
+        levels.append(tuple(level))
+        ladder.append((k, elig[k], r[1]))
+        act, n_act = nxt_act, r[0]
     if timing is not None:
         torch.cuda.synchronize()
         timing["exist"] = timing.get("exist", 0.0) + time.perf_counter() - t0
         t0 = time.perf_counter()
-    nxt = torch.zeros(N, dtype=torch.int16, device=dev)
-    cnt = torch.zeros(N, dtype=torch.int32, device=dev)
-    # each level's final positions (those whose longest match has that length), grouped by one sort
-    qpos = torch.nonzero(sel).squeeze(1)
-    qlen = length[qpos]
-    order = torch.argsort(qlen, stable=True)
-    qpos, qlen = qpos[order].to(torch.int32), qlen[order]
-    bounds = torch.searchsorted(qlen, torch.arange(len(levels) + 2, device=dev, dtype=torch.int32)).cpu().tolist()
-    batch: list = []  # list levels waiting to be counted together: (k, final positions, index)
-    batch_ev = 0
-    for k in range(1, len(levels) + 1):
-        kind, hs, nh = levels[k - 1][:3]
-        if kind == "bm":  # counted from the context ids the existence scan stored: no second query index or probe
-            _count_ids(elib, lib, tok, L, levels[k - 1], k, length, flags, grid, nxt, cnt)
-            levels[k - 1] = levels[k - 1][:3]
-            continue
-        fpos = qpos[bounds[k] : bounds[k + 1]]
-        m = fpos.numel()
-        if m == 0:
-            continue
-        if kind == "list":  # a sparse level: counted with the other list levels, one count for all
-            # its index is not checked here (no host wait per level): the batch reads every level's counters with its
-            # event total, and is counted again on indexes checked as they are built if an insert found no slot
-            vi = QueryIndex(elib, x, avail, k, fpos, compact=True, expect=m, defer=True)
-            batch.append((k, fpos, vi))
-            batch_ev += nh
-            if batch_ev >= BATCH_EVENTS:
-                _count_batch(elib, lib, tok, L, x, avail, batch, levels, flags, grid, nxt, cnt)
-                batch, batch_ev = [], 0
-            continue
-        vi = QueryIndex(elib, x, avail, k, fpos, compact=True)
-        # the level's hit positions probed against the final contexts; their hits emitted, partitioned and counted in
-        # LDS, then each final context's top entry
-        flags.zero_()
-        ev, n_ev = _scan_list(elib, tok, L, k, vi, x, hs, None, 0, flags, grid)
-        if int(flags[0].item()) & 4:
-            raise RuntimeError(f"k={k}: an emit region overflowed")
-        c = count_events(elib, lib, ev, n_ev, vi.ids, _RATIO.get(k, 1.0), presort="ctx")
-        n_ev = c.n_ev
-        EVENTS[0] += n_ev
-        del ev
-        _RATIO[k] = c.U / max(1, n_ev)
-        o_tok = torch.zeros(m, dtype=torch.int16, device=dev)
-        o_cnt = torch.zeros(m, dtype=torch.int32, device=dev)
-        if c.cb:
-            sm = summarize(elib, lib, c, vi.ids, 1)
-            rec, dist = sm.rec, sm.dist
-            o_tot = torch.empty(m, dtype=torch.int32, device=dev)
-            o_dist = torch.empty(m, dtype=torch.int32, device=dev)
-            o_tc = torch.empty(m, dtype=torch.int32, device=dev)
-            elib("ng_pos_summary", vi.ctx_of, m, 0, vi.ids, None, rec, dist, None, None, i32(1), i32(1), i32(0),
-                 o_tot, o_dist, o_tc, o_tok, o_cnt, None, None)
-            del rec, dist, o_tot, o_dist, o_tc
-        else:  # unpacked pairs: sorted by key, per-context top entry by selection
-            _top1_unpacked(elib, lib, vi, c, x, o_tok, o_cnt)
-        nxt[fpos.long()] = o_tok
-        cnt[fpos.long()] = o_cnt
-        del vi, c, o_tok, o_cnt
-    if batch:
-        _count_batch(elib, lib, tok, L, x, avail, batch, levels, flags, grid, nxt, cnt)
+    nxt = elib.fill(torch.empty(N, dtype=torch.int16, device=dev), 0)
+    cnt = elib.zeros(N, torch.int32, dev)
+    _count(elib, lib, tok, L, x, avail, levels, ladder, deep, length, flags, grid, nxt, cnt)
     if timing is not None:
         torch.cuda.synchronize()
         timing["count"] = timing.get("count", 0.0) + time.perf_counter() - t0
@@ -208,21 +184,183 @@ def longest_match(tok: torch.Tensor, x: torch.Tensor, avail: torch.Tensor, cap: 
     return length, nxt, cnt, ladder
 
 
+def _exist_list(elib: Lib, tok, L: int, x, avail, act, n_act: int, k: int, prev: tuple, length, flags, grid: int, row,
+                nxt_act) -> list:
+    """One list level of the existence phase with host reads (the device levels' counterpart): the level's row of meta,
+    its hit list last."""
+    vi = QueryIndex(elib, x, avail, k, act[:n_act], compact=True)
+    _CONTEXTS[k] = vi.n / max(1, n_act)
+    hit = elib.zeros((vi.ids + 31) // 32, torch.int32, x.device)
+    cand = prev[1] if prev[0] == "list" else _bits_list(elib, prev[1], prev[2])
+    hl, nh = _scan_list(elib, tok, L, k, vi, x, cand, hit, 1, flags, grid)
+    n_dev = torch.tensor([n_act], dtype=torch.int64, device=x.device)
+    elib("ng_act_next", act, n_dev, n_act, vi.ctx_of, hit, avail, i32(k), length, nxt_act, row, row[1:])
+    row[2:3].fill_(nh)
+    return row.cpu().tolist() + [hl]
+
+
+def _count(elib: Lib, lib: Lib, tok, L: int, x, avail, levels: list, ladder: list, deep, length, flags, grid: int, nxt,
+           cnt) -> None:
+    """The counting phase: each position's final context (of its length k) counted, its top entry to nxt / cnt. Levels are
+    counted together, their context ids offset, while the ids fit the 32-bit count and the scan regions GROUP_EVENTS: a
+    small corpus's levels cost one count's launches, not one each."""
+    matched = [m for _, _, m in ladder] + [0]
+    final = [matched[j] - matched[j + 1] for j in range(len(ladder))]  # positions whose match ends at level j + 1
+    lists = [k for k in range(1, len(levels) + 1) if levels[k - 1][0] == "list" and final[k - 1]]
+    R = emit_region(L, grid)
+    group: list = []
+    used = cap_ev = 0
+    for k in [k for k in range(1, len(levels) + 1) if levels[k - 1][0] == "bm" and final[k - 1]] + (["lists"] if lists
+                                                                                                    else []):
+        if k == "lists":
+            ids, ev = int(deep[2] / QLOAD) + 1024 + QTAIL, sum(levels[j - 1][2] for j in lists)
+            wide = lists[0] in _WIDE
+        else:
+            ids, ev = levels[k - 1][6], grid * R
+            wide = k in _WIDE
+        ids = (ids + 31) // 32 * 32  # each level's final bits start at a word
+        if wide or w_bits(ids)[1] > W_MAX:  # by the 64-bit count, alone
+            _count_wide(elib, lib, tok, L, x, avail, [k], lists, levels, length, flags, grid, nxt, cnt)
+            continue
+        if group and (w_bits(used + ids)[1] > W_MAX or cap_ev + ev > GROUP_EVENTS):
+            _count_group(elib, lib, tok, L, x, avail, group, lists, levels, deep, length, flags, grid, nxt, cnt)
+            group, used, cap_ev = [], 0, 0
+        group.append((k, used, ids))
+        used += ids
+        cap_ev += ev
+    if group:
+        _count_group(elib, lib, tok, L, x, avail, group, lists, levels, deep, length, flags, grid, nxt, cnt)
+
+
+def _count_group(elib: Lib, lib: Lib, tok, L: int, x, avail, group: list, lists: list, levels: list, deep, length, flags,
+                 grid: int, nxt, cnt) -> None:
+    """The levels of `group` ((k, first id, ids), or ("lists", ...): the list levels with final positions) in one 32-bit
+    count. A bitmap level's final contexts are marked in a bit set and its stored ids emit their events; the list levels'
+    final contexts go into one table, which their listed positions are probed against (ng_lm_index, ng_lm_lists_emit)."""
+    dev = x.device
+    N = x.numel()
+    n_ids = sum(ids for _, _, ids in group)
+    _, W = w_bits(n_ids)
+    d1 = first_digit(W)
+    # events keyed by context range only for a level by itself: several levels' id ranges hold far from equal events, and
+    # the partitions of the densest would overflow
+    mbits = key_mbits(W) if len(group) == 1 and runs_fit(n_ids, 1) else W
+    bms = [g for g in group if g[0] != "lists"]
+    total = sum(levels[k - 1][2] for k in lists) if len(bms) < len(group) else 0
+    R = emit_region(L, grid) if bms else 0
+    gl = 0
+    if total or len(bms) < len(group):
+        gl = max(1, min(grid, -(-total // 1024)))
+        if R:
+            gl = max(gl, -(-total // R))
+        R = max(R, -(-max(total, 1) // (gl * 256)) * 256)
+    nseg = len(bms) * grid + gl
+    regions = torch.empty(nseg * R, dtype=torch.int64, device=dev)
+    ev_count = torch.empty(nseg, dtype=torch.int32, device=dev)
+    dhist = torch.empty((1 << d1) * nseg, dtype=torch.int32, device=dev)
+    fid = elib.full_ones(N, torch.int32, dev)
+    bits = elib.zeros(n_ids // 32, torch.int32, dev)
+    elib.fill(flags, 0)
+    for j, (k, base, ids) in enumerate(bms):
+        _, bm, _, stored, act, ctx_of, _, n_act = levels[k - 1]
+        elib("ng_lm_final", act, n_act, ctx_of, length, i32(k), i32(base), fid, bits[base // 32 :])
+        elib("ng_scan_ids_emit", tok, L, bm, stored, bits[base // 32 :], regions[j * grid * R :], u64(R),
+             ev_count[j * grid :], flags, i32(grid), dhist[j * grid :], nseg, i32(W), i32(d1), i32(mbits),
+             u64(base << 16))
+    counters = None
+    if gl:
+        _, base, _ = group[-1]
+        k0, act0, n0 = deep
+        qcap = int(n0 / QLOAD) + 1024
+        slots = qcap + QTAIL
+        table = elib.full_ones(slots, torch.int64, dev)
+        rep = torch.empty(slots, dtype=torch.int32, device=dev)
+        counters = elib.zeros((65, 3), torch.int64, dev)
+        mixed = SimpleNamespace(cap=qcap, ids=slots, table=table, rep=rep)
+        for k in lists:
+            QueryIndex(elib, x, avail, k, act0[:n0], compact=True, expect=n0, defer=True, counters=counters[k],
+                       shared=mixed)
+        elib("ng_lm_index", x, act0, n0, length, i32(k0), table, u64(qcap), u64(slots), rep, i32(base), fid, counters)
+        rows = (ctypes.c_int64 * (3 * len(lists)))(*[v for k in lists for v in (levels[k - 1][1].data_ptr(),
+                                                                               levels[k - 1][2], k)])
+        at = len(bms) * grid
+        elib("ng_lm_lists_emit", tok, rows, i32(len(lists)), table, u64(qcap), rep, x, length, regions[at * R :], u64(R),
+             ev_count[at:], flags, i32(gl), dhist[at:], nseg, i32(W), i32(d1), i32(mbits), u64(base << 16))
+    key = tuple(k for k, _, _ in group)
+    min_pbits = 0
+    seg = (regions, R, ev_count, dhist, nseg, flags)
+    while True:
+        c = count32(elib, seg, n_ids, 1, None, None, _RATIO.get(key, 1.0), min_pbits=min_pbits, mbits=mbits)
+        got = torch.cat([c.stat[:3], flags[:1].to(torch.int64)] + ([counters.view(-1)] if gl else [])).tolist()
+        n_ev, n_u, fl, sfl = got[:4]
+        if sfl & 4:
+            raise RuntimeError(f"levels {key}: an emit region overflowed")
+        if fl & 4:
+            raise RuntimeError(f"levels {key}: a total does not fit uint32")
+        over = False
+        for k in lists if gl else ():
+            _, o, coll = got[4 + 3 * k : 7 + 3 * k]
+            if coll:
+                raise RuntimeError(f"k={k}: {coll} query positions collide with another context's key")
+            over |= o != 0
+        if over:  # an insert found no slot: the list levels by themselves, their indexes checked as they are built
+            del regions, seg, c, dhist
+            _count_wide(elib, lib, tok, L, x, avail, ["lists"], lists, levels, length, flags, grid, nxt, cnt)
+            bms_left = [g for g in group if g[0] != "lists"]
+            if bms_left:
+                _count_group(elib, lib, tok, L, x, avail, bms_left, lists, levels, deep, length, flags, grid, nxt, cnt)
+            return
+        if fl & 1 and not fl & 2 and c.pbits < pbits32_max(n_ids):  # a partition overfull: counted with a bit more
+            min_pbits = c.pbits + 1
+            continue
+        break
+    if fl & 3:  # its escape table overflowed, or no more partition bits: these levels take the 64-bit count from now on
+        del regions, seg, c, dhist
+        for k, _, _ in group:
+            _WIDE.add(lists[0] if k == "lists" else k)
+        _count_wide(elib, lib, tok, L, x, avail, [k for k, _, _ in group], lists, levels, length, flags, grid, nxt, cnt)
+        return
+    _RATIO[key] = n_u / max(1, n_ev)
+    EVENTS[0] += n_ev
+    elib("ng_lm_top1", fid, N, n_ids, c.rec, c.dist, nxt, cnt)
+
+
+def _count_wide(elib: Lib, lib: Lib, tok, L: int, x, avail, ks: list, lists: list, levels: list, length, flags, grid: int,
+                nxt, cnt) -> None:
+    """Levels by the 64-bit count: a bitmap level from its stored ids, the list levels with an index each, checked, in
+    batches."""
+    for k in ks:
+        if k != "lists":
+            level = levels[k - 1]
+            n_act = level[7]
+            _count_ids(elib, lib, tok, L, (*level[:4], level[4][:n_act], level[5][:n_act], level[6]), k, length, flags,
+                       grid, nxt, cnt)
+            continue
+        batch, ev = [], 0
+        for j in lists:
+            fpos = torch.nonzero(length == j).squeeze(1).to(torch.int32)
+            batch.append((j, fpos, QueryIndex(elib, x, avail, j, fpos, compact=True)))
+            ev += levels[j - 1][2]
+            if ev >= BATCH_EVENTS or j == lists[-1]:
+                _count_batch(elib, lib, tok, L, x, avail, batch, levels, flags, grid, nxt, cnt)
+                batch, ev = [], 0
+
+
 SCAN_BLOCKS_PER_CU = 32  # scan blocks per compute unit
 TOK1_GRID = 2048  # level 1's scan blocks (each ORs its hit words into the level's once)
 EVENTS = [0]  # (context, next) events the last longest_match counted (its counting phase), for its timing dict
 DEVICE_LEVELS = True  # the existence phase's levels after the second list level run without host syncs
 LONG_FIRST = 8  # the device levels try level cap first when at least this many levels lie between
+GROUP_EVENTS = 1 << 26  # bitmap levels counted together until their scan regions hold this many events
 BATCH_EVENTS = 1 << 28  # list levels counted together until their listed positions reach this
 LIST_DIV = 64  # a level's hits go to a position list once fewer than L / LIST_DIV (8 B each against L / 8 bitmap bytes)
 
 
 def _exist_device(elib: Lib, tok, L: int, x, avail, act, k0: int, cap: int, cand, length, flags, grid: int):
-    """Levels k0..cap of the existence phase as one stream of launches with no host sync (ng_query_index_dev,
-    ng_scan_list_dev, ng_seg_offsets / ng_seg_gather, ng_act_next), every buffer sized by level k0's active
-    positions (act, already those with avail >= k0) and candidates (cand: the corpus positions that matched k0 - 1),
-    which bound every later level's. One sync at the end reads each level's sizes; the levels are those whose active
-    list was not empty, as the host loop's. Returns [(k, hit list, its length, matched positions)].
+    """Levels k0..cap of the existence phase launched by one call with no host sync (ng_lm_levels), every buffer sized by
+    level k0's active positions (act, all with avail >= k0) and candidates (cand: the corpus positions that matched
+    k0 - 1), which bound every later level's. One sync at the end reads each level's sizes; the levels are those whose
+    active list was not empty, as the host loop's. Returns [(k, hit list, its length, matched positions)].
 
     With LONG_FIRST or more levels to go, level `cap` is tried first (the cap round): a position whose cap-token
     context occurs matches every level below it too (a context's suffixes occur wherever it does), so it is done at
@@ -233,91 +371,33 @@ def _exist_device(elib: Lib, tok, L: int, x, avail, act, k0: int, cap: int, cand
     n0, nc0 = int(act.numel()), int(cand.numel())
     qcap = int(n0 / QLOAD) + 1024
     slots = qcap + QTAIL
-    table = torch.empty(slots, dtype=torch.int64, device=dev)
+    table = elib.full_ones(slots, torch.int64, dev)
     rep = torch.empty(slots, dtype=torch.int32, device=dev)
-    ctx_of = torch.empty(max(n0, 1), dtype=torch.int32, device=dev)
-    hit = torch.empty((slots + 31) // 32, dtype=torch.int32, device=dev)
-    acts = [act.contiguous(), torch.empty(max(n0, 1), dtype=torch.int32, device=dev)]
+    lvl = elib.fill(torch.empty((slots + 7) // 8 * 8, dtype=torch.uint8, device=dev), 0)
+    ctx_of, act_a, act_b = (torch.empty(max(n0, 1), dtype=torch.int32, device=dev) for _ in range(3))
     nlev = cap - k0 + 1
-    counters = torch.zeros((nlev, 3), dtype=torch.int64, device=dev)
-    sizes = torch.zeros((nlev, 3), dtype=torch.int64, device=dev)  # per level: active, matched, kept for the next
-    g = max(1, min(grid, -(-max(nc0, 1) // 256)))
-    R = -(-max(nc0, 1) // (g * 256)) * 256
-    regions = torch.empty(g * R, dtype=torch.int64, device=dev)
-    ev_count = torch.empty(g, dtype=torch.int32, device=dev)
-    n_act = torch.tensor([n0], dtype=torch.int64, device=dev)
-    n_cand = torch.tensor([nc0], dtype=torch.int64, device=dev)
-    flags.zero_()
     first = cap - k0 >= LONG_FIRST
-    if first:  # the cap round: the positions matching level cap are done; the others go on from level k0
-        counters_cap = torch.zeros(3, dtype=torch.int64, device=dev)
-        split = torch.zeros(2, dtype=torch.int64, device=dev)  # positions going on, positions done at length cap
-        elib("ng_query_index_dev", x, avail, acts[0], n_act, n0, i32(cap), table, u64(qcap), u64(slots), rep, ctx_of,
-             counters_cap)
-        hit.zero_()
-        elib("ng_scan_list_dev", tok, i32(cap), cand, n_cand, nc0, table, u64(qcap), rep, x, hit, i32(1), regions,
-             u64(R), ev_count, flags, i32(g), u64(0))
-        offs = torch.empty(g + 1, dtype=torch.int64, device=dev)
-        elib("ng_seg_offsets", ev_count, g, offs)
-        hl_cap = torch.empty(max(nc0, 1), dtype=torch.int64, device=dev)
-        elib("ng_seg_gather", regions, None, u64(R), None, ev_count, g, offs, hl_cap, None)
-        elib("ng_act_split", acts[0], n_act, n0, ctx_of, hit, i32(cap), length, acts[1], split[0:1], split[1:2])
-        nh_cap, n_act = offs[g:], split[0:1]
-        acts.reverse()
-    out = []
-    for j, k in enumerate(range(k0, cap if first else cap + 1)):
-        cur, nxt = acts[j % 2], acts[(j + 1) % 2]
-        sizes[j, 0:1].copy_(n_act)
-        elib("ng_query_index_dev", x, avail, cur, n_act, n0, i32(k), table, u64(qcap), u64(slots), rep, ctx_of,
-             counters[j])
-        hit.zero_()
-        elib("ng_scan_list_dev", tok, i32(k), cand, n_cand, nc0, table, u64(qcap), rep, x, hit, i32(1), regions,
-             u64(R), ev_count, flags, i32(g), u64(0))
-        offs = torch.empty(g + 1, dtype=torch.int64, device=dev)
-        elib("ng_seg_offsets", ev_count, g, offs)
-        hl = torch.empty(max(nc0, 1), dtype=torch.int64, device=dev)
-        elib("ng_seg_gather", regions, None, u64(R), None, ev_count, g, offs, hl, None)
-        elib("ng_act_next", cur, n_act, n0, ctx_of, hit, avail, i32(k), length, nxt, sizes[j, 2:3], sizes[j, 1:2])
-        out.append((k, hl, offs[g:]))
-        cand, n_cand, n_act = hl, offs[g:], sizes[j, 2:3]
-    if first:
-        out.append((cap, hl_cap, nh_cap))
-        counters = torch.cat([counters, counters_cap[None]])
-        sizes[-1, 1:2].copy_(split[1:2])
-    host = sizes.cpu().tolist()
-    nhs = torch.cat([o for _, _, o in out]).cpu().tolist()
-    c = counters.cpu()
-    if int(flags[0].item()) & 4:
-        raise RuntimeError(f"levels {k0}..{cap}: an emit region overflowed")
-    if int(c[:, 1].max()):
+    hl = torch.empty((nlev, max(nc0, 1)), dtype=torch.int64, device=dev)
+    meta = elib.zeros((nlev + 1, 6), torch.int64, dev)
+    elib("ng_lm_levels", tok, x, avail, i32(k0), i32(cap), i32(int(first)), act, n0, act_a, act_b, cand, nc0, table,
+         u64(qcap), u64(slots), rep, ctx_of, lvl, hl, length, meta, flags, i32(grid))
+    host = meta.cpu().tolist()
+    if any(r[4] for r in host[:nlev]):
         raise RuntimeError(f"levels {k0}..{cap}: a query index was too small for its contexts")
-    if int(c[:, 2].max()):
+    if any(r[5] for r in host[:nlev]):
         raise RuntimeError(f"levels {k0}..{cap}: query positions collide with another context's key")
-    done = host[-1][1] if first else 0  # the positions done at length cap: active and matched at every level
-    if first:  # level cap's active positions: the others' that reached it, and the cap round's
-        host[-1][0] = host[-2][2] if len(host) > 1 else 0
+    going, done = (host[-1][0], host[-1][1]) if first else (n0, 0)  # done: the positions done at length cap
     res = []
-    for (k, hl, _), nh, (n_k, matched, _) in zip(out, nhs, host):
-        if k < cap:
-            n_k, matched = n_k + done, matched + done
-        else:
-            n_k += done if first else 0
-        if n_k == 0:
+    active = going
+    for j, k in enumerate(range(k0, cap + 1)):
+        kept, matched, nh = host[j][:3]
+        if first and k == cap:  # its trial took place first: the others that reached it did not match
+            matched = 0
+        if active + done == 0:
             break
-        res.append((k, hl[:nh], nh, matched))
+        res.append((k, hl[j, :nh], nh, matched + done))
+        active = kept
     return res
-
-
-def _tok1_index(x: torch.Tensor, act: torch.Tensor) -> SimpleNamespace:
-    """Level 1's index without a table: each listed position's context id is its token (x[act], ids 0..65535), and
-    `member` (int32 [2048]) holds bit t for each token t among them."""
-    dev = x.device
-    ctx_of = x[act.long()].to(torch.int32) & 0xFFFF
-    seen = torch.zeros(65536, dtype=torch.bool, device=dev)
-    seen[ctx_of.long()] = True
-    w = (seen.view(2048, 32).to(torch.int64) << torch.arange(32, device=dev)).sum(1)
-    member = torch.where(w >= 1 << 31, w - (1 << 32), w).to(torch.int32)  # the words' bits, as int32
-    return SimpleNamespace(ctx_of=ctx_of, ids=65536, member=member)
 
 
 def _count_ids(elib: Lib, lib: Lib, tok, L: int, level: tuple, k: int, length, flags, grid: int, nxt, cnt) -> None:
@@ -340,20 +420,10 @@ def _count_ids(elib: Lib, lib: Lib, tok, L: int, level: tuple, k: int, length, f
     R = emit_region(L, grid)
     regions = torch.empty(grid * R, dtype=torch.int64, device=dev)
     ev_count = torch.empty(grid, dtype=torch.int32, device=dev)
-    _, W = w_bits(n_ids)
-    if W <= W_MAX and k not in _WIDE:  # the 32-bit count (pairs32.hip), as the level pipeline's
-        d1 = first_digit(W)
-        dhist = torch.empty((1 << d1) * grid, dtype=torch.int32, device=dev)
-        flags.zero_()
-        elib("ng_scan_ids_emit", tok, L, bm, ids, final, regions, u64(R), ev_count, flags, i32(grid), dhist, grid,
-             i32(W), i32(d1), i32(key_mbits(W) if runs_fit(n_ids, 1) else W))
-        if _count32_final(elib, (regions, R, ev_count, dhist, grid, flags), n_ids, k, fids, fpos, m, nxt, cnt):
-            return
-        _WIDE.add(k)  # its escape table overflowed: this level takes the 64-bit count from now on
     dhist = torch.empty(256 * grid, dtype=torch.int32, device=dev)
     flags.zero_()
     elib("ng_scan_ids_emit", tok, L, bm, ids, final, regions, u64(R), ev_count, flags, i32(grid), dhist, grid, i32(0),
-         i32(0), i32(0))
+         i32(0), i32(0), u64(0))
     try:  # the scan's flags read with the event total
         c = count_events(elib, lib, None, 0, n_ids, _RATIO.get(k, 1.0),
                          seg=(regions, R, ev_count, dhist, grid, flags), presort="ctx")
@@ -373,40 +443,6 @@ def _count_ids(elib: Lib, lib: Lib, tok, L: int, level: tuple, k: int, length, f
         _top1_unpacked(elib, lib, SimpleNamespace(ctx_of=fids, ids=n_ids), c, None, o_tok, o_cnt)
     nxt[fpos] = o_tok
     cnt[fpos] = o_cnt
-
-
-def _count32_final(elib: Lib, seg: tuple, n_ids: int, k: int, fids, fpos, m: int, nxt, cnt) -> bool:
-    """The 32-bit count of a level's final contexts' events (seg: ng_scan_ids_emit's W-bit regions), their top entry
-    gathered to the final positions; an overfull partition is counted again with one more partition bit. False (the
-    caller takes the 64-bit count) when the escape table overflowed."""
-    dev = fids.device
-    min_pbits = 0
-    while True:
-        c = count32(elib, seg, n_ids, 1, None, None, _RATIO.get(k, 1.0), min_pbits=min_pbits,
-                    mbits=key_mbits(w_bits(n_ids)[1]) if runs_fit(n_ids, 1) else None)
-        n_ev, n_u, fl, scan = c.stat[:4].cpu().tolist()
-        if int(seg[5][0].item()) & 4:
-            raise RuntimeError(f"k={k}: an emit region overflowed")
-        if fl & 4:
-            raise RuntimeError(f"k={k}: a total does not fit uint32")
-        if fl & 2:
-            return False
-        if fl & 1 and c.pbits < pbits32_max(n_ids):
-            min_pbits = c.pbits + 1
-            continue
-        if fl & 1:
-            return False
-        break
-    _RATIO[k] = n_u / max(1, n_ev)
-    EVENTS[0] += n_ev
-    o = [torch.empty(m, dtype=torch.int32, device=dev) for _ in range(3)]
-    o_tok = torch.zeros(m, dtype=torch.int16, device=dev)
-    o_cnt = torch.zeros(m, dtype=torch.int32, device=dev)
-    elib("ng_pos_summary", fids, m, 0, n_ids, None, c.rec, c.dist, None, None, i32(1), i32(1), i32(0), o[0], o[1],
-         o[2], o_tok, o_cnt, None, None)
-    nxt[fpos] = o_tok
-    cnt[fpos] = o_cnt
-    return True
 
 
 def _bits_list(elib: Lib, bm: torch.Tensor, n: int) -> torch.Tensor:
