@@ -368,22 +368,29 @@ def count32(elib: Lib, seg: tuple, n_ids: int, ktop: int, lookups: tuple | None,
         n_events = int(ev_tot.item())
     # events keyed by context range (M < W) fill only the partitions of the used share of the id bits
     used = n_ids / (1 << idb) if M < W else 1.0
-    pbits = max(d1 + 1, W - 31, PART_MIN_BITS if lookups is not None else 0, min_pbits,
-                math.ceil(math.log2(max(1.0, n_events * ratio / P32_TARGET / used))))
+    pbits = max(d1, W - 31, min_pbits, math.ceil(math.log2(max(1.0, n_events * ratio / P32_TARGET / used))))
+    # a level of few events needs no partition below the first pass's digit (2^8 partitions, one per compute unit): no
+    # second pass, and the lookups are sorted by 8 bits. One that needs more takes PART_MIN_BITS at least where it has
+    # lookups (a block's several smaller partitions even out: 2^9 counted 4.2M tokens' bigrams in 112 us, 2^11 in 89).
+    # Seven levels of 64M corpus tokens, five of them with few events: 5.72 ms a build with 2^11 always, 5.38 here
+    if pbits > d1 and lookups is not None:
+        pbits = max(pbits, PART_MIN_BITS)
     pbits = min(pbits, pbits32_max(n_ids))
     d2 = pbits - d1
     e0, e1 = event("partition", cap)
     e0.record()
-    ev32b = torch.empty(max(cap, 1), dtype=torch.int32, device=dev)
     P = 1 << pbits
     start = torch.empty(P + 1, dtype=torch.int64, device=dev)
     if W <= W_MAX:
         ev1 = torch.empty(max(cap, 1), dtype=torch.int32, device=dev)
         elib("ng_seg_scatter_narrow", regions, u64(R), None, ev_count, dpre, nseg, i32(W - d1), i32(d1), ev1, u64(cap))
-        elib.cub("ng_msd_pass", ev1, dpre, nseg, i32(d1), ev_tot, u64(cap), i32(W - pbits), i32(d2), ev32b, start)
+        ev32b = torch.empty(max(cap, 1), dtype=torch.int32, device=dev) if d2 else ev1
+        elib.cub("ng_msd_pass", ev1, dpre, nseg, i32(d1), ev_tot, u64(cap), i32(W - pbits), i32(d2),
+                 ev32b if d2 else None, start)
     else:  # wide keys: 64 bits through the first pass, narrowed by the second
         ev1 = torch.empty(max(cap, 1), dtype=torch.int64, device=dev)
         elib("ng_seg_scatter", regions, u64(R), None, ev_count, dpre, nseg, i32(W - d1), i32(d1), ev1, u64(cap))
+        ev32b = torch.empty(max(cap, 1), dtype=torch.int32, device=dev)
         elib.cub("ng_msd_pass_narrow", ev1, dpre, nseg, i32(d1), ev_tot, u64(cap), i32(W - pbits), i32(d2), ev32b,
                  start)
     del ev1, dpre
