@@ -272,6 +272,16 @@ __device__ __forceinline__ i64 ctx_find_insert(u64* ck, u64 ccap, u64 key, u32* 
     return -1;
 }
 
+// One lane of a block per key: claim (LDS, ELECT_SLOTS u64, EMPTY-filled) takes the first lane's key at its place, and a
+// lane that finds its own key there is a duplicate (false); a lane that finds another key there is not held back. Where
+// the threads of a launch start on an empty table together, every lane of a frequent key would try the compare-and-swap
+// of its slot, and same-address atomics run at about 80 M/s: with one lane a block per key the later ones find it there.
+#define ELECT_SLOTS 512
+__device__ __forceinline__ bool elect(u64* claim, u64 key) {
+    const u64 prev = atomicCAS((unsigned long long*)&claim[(u32)key & (ELECT_SLOTS - 1)], EMPTY, key);
+    return prev != key;
+}
+
 // The slot of `key` in such a table, or -1.
 __device__ __forceinline__ i64 ctx_find(const u64* __restrict__ ck, u64 ccap, u64 key) {
     u64 s = __umul64hi(key, ccap);
