@@ -129,6 +129,7 @@ def bench_c2(steps: int, warmup: int, with_cpu: bool) -> dict:
     cold_ms = None
     for step in range(warmup + steps):
         ct = CountTable.from_device(tok, sizes, starts, levels, sizing=sizing)
+        ct.timed = True
         torch.cuda.synchronize()
         t0 = time.perf_counter()
         ct.build()
@@ -635,6 +636,7 @@ def main() -> None:
         torch.cuda.synchronize()
         cold[label] = 1e3 * (time.perf_counter() - t0)
     cold["reruns"] = cb.engine.reruns
+    cb.engine.timed = True  # kernel_events below
     log("cold:", json.dumps(cold))
     # one untimed build with hit counts: the hits E of the roofline (deterministic, the same every step)
     cb.counts(x, tgt, avail, stats=True)

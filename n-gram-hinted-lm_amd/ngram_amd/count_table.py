@@ -74,6 +74,8 @@ class CountTable:
     """Exact next-token counts of every k-context (k of `levels`) in the training shards (count_table.rs), on the GPU:
     create before the clock, build on it, query the validation tokens (inputs + the last target) after it."""
 
+    timed = False  # whether builds and queries record `events` (each costs about 5 us of the stream)
+
     def __init__(self):
         raise TypeError("use CountTable.create(files, levels, threads, cpus)")
 
@@ -161,6 +163,9 @@ class CountTable:
             self.tables.append(self._build_level(k))
 
     def _timed(self, name: str, k: int):
+        """Timing events around a launch, kept in `events`, where the table is `timed`."""
+        if not self.timed:
+            return P.NO_EVENTS
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         self.events.append((name, k, e0, e1))
         return e0, e1

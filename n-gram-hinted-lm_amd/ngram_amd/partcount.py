@@ -38,12 +38,16 @@ def emit_region(L: int, grid: int) -> int:
     return -(-L // per) * 8192
 
 
-def _no_event(name: str, n: int):
-    class _E:
-        def record(self):
-            pass
+class _NoEvent:
+    def record(self) -> None:
+        pass
 
-    return _E(), _E()
+
+NO_EVENTS = (_NoEvent(), _NoEvent())
+
+
+def _no_event(name: str, n: int):
+    return NO_EVENTS
 
 
 class _HostRead:
