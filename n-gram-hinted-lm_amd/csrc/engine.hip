@@ -1758,11 +1758,9 @@ __global__ void __launch_bounds__(256) lm_scan_k(const u16* __restrict__ tok, co
         __syncthreads();
         const u32 m = s_n;  // block-uniform
         if (m > LM_STAGE - 1024 || c0 + stride >= n) {
-            if (threadIdx.x == 0) {
-                s_base = m ? atomicAdd((unsigned long long*)n_hits, (unsigned long long)m) : 0;
-                s_n = 0;
-            }
-            __syncthreads();
+            if (threadIdx.x == 0) s_base = m ? atomicAdd((unsigned long long*)n_hits, (unsigned long long)m) : 0;
+            __syncthreads();  // every wave has read s_n: only now is it reset, before the next round's first barrier
+            if (threadIdx.x == 0) s_n = 0;
             for (u32 i = threadIdx.x; i < m; i += 256) hl[s_base + i] = s_hit[i];
         }
     }
