@@ -75,8 +75,9 @@ def longest_match(tok: torch.Tensor, x: torch.Tensor, avail: torch.Tensor, cap: 
     act = torch.empty(max(N, 1), dtype=torch.int32, device=dev)
     mask = None
     if query is not None:
-        mask = query if query.dtype in (torch.bool, torch.uint8) else query.bool()
-        mask = mask.expand(N).contiguous().view(torch.uint8)
+        # torch combines the two: it refuses a mask in host memory, which the kernel would read through its address, and
+        # one of another shape
+        mask = torch.ne((avail >= 1) & query, 0).expand(N).view(torch.uint8)
     elib("ng_lm_select", avail, mask, N, i32(cap), act, rows[0], hist)
     # each level's hit set (the corpus positions whose k-context is a query context of the level): a bitmap while
     # dense, then, once sparse, a list of positions, which the next level scans instead of every bitmap word
