@@ -174,11 +174,15 @@ int ng_scan_tok1(const uint16_t* tok, ng_i64 L, const uint32_t* member, uint32_t
                  uint32_t* ids, int grid, void* stream);
 /* a level's counting scan from ng_scan_exist's ids (NULL: ng_scan_tok1's level, the id at p being tok[p - 1]): each
  * position set in bm whose context's bit is set in `final` emits its (id << 16 | tok[p]) event as ng_scan_emit's (regions, ev_count, dhist; wbits 0: mix64 with the top 8
- * bits' histogram, wbits 17..63: kmix(key, wbits, mbits) with the top dbits bits', dbits <= 10; key_add added to each key
- * first: a context-id offset << 16); L a multiple of 32, tok 8-byte and ids 16-byte aligned */
+ * bits' histogram, wbits 17..63: kmix(key, wbits, mbits) with the top dbits bits', dbits <= 10); L a multiple of 32, tok
+ * 8-byte and ids 16-byte aligned */
 int ng_scan_ids_emit(const uint16_t* tok, ng_i64 L, const uint32_t* bm, const uint32_t* ids, const uint32_t* final,
                      ng_u64* ev, ng_u64 region, uint32_t* ev_count, uint32_t* flags, int grid, uint32_t* dhist,
-                     ng_i64 dstride, int wbits, int dbits, int mbits, ng_u64 key_add, void* stream);
+                     ng_i64 dstride, int wbits, int dbits, int mbits, void* stream);
+/* ng_scan_ids_emit with key_add (a context-id offset << 16) added to each pair key first */
+int ng_scan_ids_emit_at(const uint16_t* tok, ng_i64 L, const uint32_t* bm, const uint32_t* ids, const uint32_t* final,
+                        ng_u64* ev, ng_u64 region, uint32_t* ev_count, uint32_t* flags, int grid, uint32_t* dhist,
+                        ng_i64 dstride, int wbits, int dbits, int mbits, ng_u64 key_add, void* stream);
 /* bit ids[i] of the u32 words bits set for each ids[i] >= 0 (bits zeroed by the caller) */
 int ng_mark_bits(const int* ids, ng_i64 n, uint32_t* bits, void* stream);
 /* a split table's occupied slots appended to (out_k, out_c) from *counter (zeroed by the caller) */
@@ -211,10 +215,25 @@ int ng_query_index(const uint16_t* x, const int* avail, const int* pos, ng_i64 n
 int ng_query_index_shrink(const ng_u64* old_t, const uint32_t* old_rep, ng_u64 old_slots, ng_u64* table, ng_u64 cap,
                           ng_u64 slots, uint32_t* rep, int* ctx_of, ng_i64 n, int* remap, ng_u64* counters,
                           void* stream);
+/* the query index of pos[0..*n_dev) (compact ctx_of; n_max >= *n_dev sizes the grid) with no host sync: the table
+ * is EMPTY-filled here, counters[1] / counters[2] added to as ng_query_index's, contexts not counted */
+int ng_query_index_dev(const uint16_t* x, const int* avail, const int* pos, const ng_u64* n_dev, ng_i64 n_max, int k,
+                       ng_u64* table, ng_u64 cap, ng_u64 slots, uint32_t* rep, int* ctx_of, ng_u64* counters,
+                       void* stream);
 /* the longest match's active list one level on: entries i < *n_dev of act whose context's hit bit is set get
  * length[act[i]] = k and, with avail >= k + 1, go to act_out (*n_out, *matched added to) */
 int ng_act_next(const int* act, const ng_u64* n_dev, ng_i64 n_max, const int* ctx_of, const uint32_t* hit,
                 const int* avail, int k, int* length, int* act_out, ng_u64* n_out, ng_u64* matched, void* stream);
+/* the longest match's active list split at level k: entries i < *n_dev of act whose context's hit bit is set get
+ * length[act[i]] = k (*matched added to); the others go to act_out (*n_out added to) */
+int ng_act_split(const int* act, const ng_u64* n_dev, ng_i64 n_max, const int* ctx_of, const uint32_t* hit, int k,
+                 int* length, int* act_out, ng_u64* n_out, ng_u64* matched, void* stream);
+/* ng_scan_sink's list scan over the first *n_dev entries of plist (n_max >= *n_dev), with no host sync; region >=
+ * ceil(n_max / (grid * 256)) * 256 */
+int ng_scan_list_dev(const uint16_t* tok, int k, const ng_u64* plist, const ng_u64* n_dev, ng_i64 n_max,
+                     const ng_u64* vt, ng_u64 vcap, const uint32_t* vrep, const uint16_t* x, uint32_t* hit, int what,
+                     ng_u64* ev, ng_u64 region, uint32_t* ev_count, uint32_t* flags, int grid, ng_u64 key_add,
+                     void* stream);
 /* the longest match's host loop (ngram_amd/longest.py): the queried positions (avail >= 1, mask[i] unless mask is NULL)
  * listed and counted by min(avail, cap); level 1's token index; the deep levels k0..cap launched together (meta u64
  * [cap - k0 + 2][6]: per level the positions kept, matched, corpus hits, ng_query_index's counters; the last row level

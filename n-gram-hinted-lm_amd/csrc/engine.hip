@@ -962,9 +962,9 @@ static inline bool emit_mode_ok(int wbits, int dbits, int& mbits) {
 // histogram of the top 8 bits; wbits in [17, 63]: kmix(pair key, wbits, mbits) (context ids below 2^(wbits - 16);
 // part.h; mbits 0: wbits) with a histogram of the top dbits bits (1 <= dbits <= 10), the 32-bit count's events. key_add:
 // added to each pair key first (a context-id offset << 16: several levels counted in one id space).
-extern "C" int ng_scan_ids_emit(const u16* tok, i64 L, const u32* bm, const u32* ids, const u32* final, u64* ev,
-                                u64 region, u32* ev_count, u32* flags, int grid, u32* dhist, i64 dstride, int wbits,
-                                int dbits, int mbits, u64 key_add, void* stream) {
+extern "C" int ng_scan_ids_emit_at(const u16* tok, i64 L, const u32* bm, const u32* ids, const u32* final, u64* ev,
+                                   u64 region, u32* ev_count, u32* flags, int grid, u32* dhist, i64 dstride, int wbits,
+                                   int dbits, int mbits, u64 key_add, void* stream) {
     if (grid <= 0 || region == 0 || region > 0xFFFFFFFFull || (dhist && dstride < grid)) return -1;
     if (!emit_mode_ok(wbits, dbits, mbits)) return -1;
     if ((L & 31) || ((uintptr_t)tok & 7) || ((uintptr_t)ids & 15)) return -1;  // the kernel's vector loads
@@ -979,6 +979,14 @@ extern "C" int ng_scan_ids_emit(const u16* tok, i64 L, const u32* bm, const u32*
     const EmitSink sk{ev, region, ev_count, 0, nullptr, dhist, dstride, key_add, wbits, dbits, mbits};
     scan_ids_k<<<grid, 256, 0, st>>>(tok, L, bm, ids, final, sk, flags);
     return (int)hipGetLastError();
+}
+
+// ng_scan_ids_emit_at with no offset.
+extern "C" int ng_scan_ids_emit(const u16* tok, i64 L, const u32* bm, const u32* ids, const u32* final, u64* ev,
+                                u64 region, u32* ev_count, u32* flags, int grid, u32* dhist, i64 dstride, int wbits,
+                                int dbits, int mbits, void* stream) {
+    return ng_scan_ids_emit_at(tok, L, bm, ids, final, ev, region, ev_count, flags, grid, dhist, dstride, wbits, dbits,
+                               mbits, 0, stream);
 }
 
 // bits (u32 words, zeroed by the caller): bit ids[i] set for each ids[i] >= 0, i < n.
@@ -1038,6 +1046,22 @@ extern "C" int ng_scan_emit_list(const u16* tok, const u64* plist, const u64* n_
     hipStream_t st = (hipStream_t)stream;
     LEVEL_DISPATCH(k, (scan_list_k<K, EmitSink><<<grid, 256, 0, st>>>(tok, plist, 0, k, vt, vcap, vrep, x, sk, flags, n_dev,
                                                                      bm_out)));
+    return (int)hipGetLastError();
+}
+
+// The list scan of ng_scan_sink over the first *n_dev entries of plist (n_max >= *n_dev; a device-side count, so no
+// host sync): hit bits and events (positions, what 1, or mixed pair keys, what 0) as ng_scan_sink's;
+// region >= ceil(n_max / (grid * 256)) * 256.
+extern "C" int ng_scan_list_dev(const u16* tok, int k, const u64* plist, const u64* n_dev, i64 n_max, const u64* vt,
+                                u64 vcap, const u32* vrep, const u16* x, u32* hit, int what, u64* ev, u64 region,
+                                u32* ev_count, u32* flags, int grid, u64 key_add, void* stream) {
+    if (grid <= 0 || !n_dev || !ev || (what != 0 && what != 1) || region == 0 || region > 0xFFFFFFFFull ||
+        (u64)n_max > (u64)grid * region)
+        return -1;
+    const EmitSink sk{ev, region, ev_count, what, hit, nullptr, 0, key_add};
+    hipStream_t st = (hipStream_t)stream;
+    LEVEL_DISPATCH(k, (scan_list_k<K, EmitSink><<<grid, 256, 0, st>>>(tok, plist, n_max, k, vt, vcap, vrep, x, sk, flags,
+                                                                     n_dev, nullptr)));
     return (int)hipGetLastError();
 }
 
@@ -1547,9 +1571,11 @@ extern "C" int ng_query_index(const u16* x, const int* avail, const int* pos, i6
 
 namespace {
 // One step of the longest match's active list: entry i (i < *n_dev) of act whose context (ctx_of[i]) has its hit bit
-// set matched level k (length[act[i]] = k); those with avail >= k + 1 go on to act_out. Each thread takes 4 entries; a
-// block counts its kept entries and matches and takes its place in act_out with one atomic each (a counter bumped per
-// entry or per wave would serialize).
+// set matched level k (length[act[i]] = k); those with avail >= k + 1 go on to act_out. SPLIT: the entries that did
+// not match go on instead (the matched ones are done at length k). Each thread takes 4 entries; a block counts its
+// kept entries and matches and takes its place in act_out with one atomic each (a counter bumped per entry or per
+// wave would serialize).
+template <bool SPLIT>
 __global__ void __launch_bounds__(256) act_next_k(const int* __restrict__ act, const u64* __restrict__ n_dev,
                                                   const int* __restrict__ ctx_of, const u32* __restrict__ hit,
                                                   const int* __restrict__ avail, int k, int* __restrict__ length,
@@ -1573,7 +1599,9 @@ __global__ void __launch_bounds__(256) act_next_k(const int* __restrict__ act, c
             if (c >= 0 && ((hit[c >> 5] >> (c & 31)) & 1u)) {
                 length[a[q]] = k;
                 ++nm;
-                keep[q] = avail[a[q]] >= k + 1;
+                keep[q] = !SPLIT && avail[a[q]] >= k + 1;
+            } else {
+                keep[q] = SPLIT;
             }
         }
         nk += keep[q];
@@ -1610,6 +1638,23 @@ __global__ void __launch_bounds__(256) act_next_k(const int* __restrict__ act, c
 }
 }  // namespace
 
+// The query index of the positions pos[0..*n_dev) (n_max >= *n_dev sizes the grid), compact ctx_of, without a host
+// sync: the table (cap + tail = slots) is EMPTY-filled here; counters[1] (a table too small) and
+// counters[2] (hashed keys that collided, k > 4) are added to, as ng_query_index's; the contexts are not counted.
+extern "C" int ng_query_index_dev(const u16* x, const int* avail, const int* pos, const u64* n_dev, i64 n_max, int k,
+                                  u64* table, u64 cap, u64 slots, u32* rep, int* ctx_of, u64* counters,
+                                  void* stream) {
+    if (cap == 0 || slots <= cap || slots > (1ull << 31) || !n_dev || !pos || n_max < 0) return -1;
+    hipStream_t st = (hipStream_t)stream;
+    fill_u32_n((u32*)table, 0xFFFFFFFFu, (i64)(2 * slots), st);
+    if (n_max == 0) return (int)hipGetLastError();
+    LEVEL_DISPATCH(k, (qindex_insert_k<K><<<grid_for(n_max, 256), 256, 0, st>>>(x, avail, pos, n_max, k, table, cap, slots,
+                                                                                rep, ctx_of, 1, counters, n_dev)));
+    if (k > 4)
+        qindex_verify_k<<<grid_for(n_max, 256), 256, 0, st>>>(x, pos, n_max, k, ctx_of, 1, rep, counters + 2, n_dev);
+    return (int)hipGetLastError();
+}
+
 // The longest match's active list, one level on: see act_next_k. n_out and matched are added to (zero them first);
 // act_out holds at least *n_dev entries; n_max >= *n_dev sizes the grid.
 extern "C" int ng_act_next(const int* act, const u64* n_dev, i64 n_max, const int* ctx_of, const u32* hit,
@@ -1617,8 +1662,19 @@ extern "C" int ng_act_next(const int* act, const u64* n_dev, i64 n_max, const in
                            void* stream) {
     if (!n_dev || n_max < 0) return -1;
     if (n_max > 0)
-        act_next_k<<<(int)((n_max + 1023) / 1024), 256, 0, (hipStream_t)stream>>>(
+        act_next_k<false><<<(int)((n_max + 1023) / 1024), 256, 0, (hipStream_t)stream>>>(
             act, n_dev, ctx_of, hit, avail, k, length, act_out, n_out, matched);
+    return (int)hipGetLastError();
+}
+
+// The longest match's active list split at level k (see act_next_k): entries whose context's hit bit is set get
+// length k and are done; the others go to act_out. n_out and matched are added to (zero them first).
+extern "C" int ng_act_split(const int* act, const u64* n_dev, i64 n_max, const int* ctx_of, const u32* hit, int k,
+                            int* length, int* act_out, u64* n_out, u64* matched, void* stream) {
+    if (!n_dev || n_max < 0) return -1;
+    if (n_max > 0)
+        act_next_k<true><<<(int)((n_max + 1023) / 1024), 256, 0, (hipStream_t)stream>>>(
+            act, n_dev, ctx_of, hit, nullptr, k, length, act_out, n_out, matched);
     return (int)hipGetLastError();
 }
 

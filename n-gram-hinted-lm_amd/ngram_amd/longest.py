@@ -265,7 +265,7 @@ def _count_group(elib: Lib, lib: Lib, tok, L: int, x, avail, group: list, lists:
     for j, (k, base, ids) in enumerate(bms):
         _, bm, _, stored, act, ctx_of, _, n_act = levels[k - 1]
         elib("ng_lm_final", act, n_act, ctx_of, length, i32(k), i32(base), fid, bits[base // 32 :])
-        elib("ng_scan_ids_emit", tok, L, bm, stored, bits[base // 32 :], regions[j * grid * R :], u64(R),
+        elib("ng_scan_ids_emit_at", tok, L, bm, stored, bits[base // 32 :], regions[j * grid * R :], u64(R),
              ev_count[j * grid :], flags, i32(grid), dhist[j * grid :], nseg, i32(W), i32(d1), i32(mbits),
              u64(base << 16))
     counters = None
@@ -424,7 +424,7 @@ def _count_ids(elib: Lib, lib: Lib, tok, L: int, level: tuple, k: int, length, f
     dhist = torch.empty(256 * grid, dtype=torch.int32, device=dev)
     flags.zero_()
     elib("ng_scan_ids_emit", tok, L, bm, ids, final, regions, u64(R), ev_count, flags, i32(grid), dhist, grid, i32(0),
-         i32(0), i32(0), u64(0))
+         i32(0), i32(0))
     try:  # the scan's flags read with the event total
         c = count_events(elib, lib, None, 0, n_ids, _RATIO.get(k, 1.0),
                          seg=(regions, R, ev_count, dhist, grid, flags), presort="ctx")

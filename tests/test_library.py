@@ -110,6 +110,16 @@ def declared_arity(header: str) -> dict[str, int]:
     return out
 
 
+def test_entry_points_keep_their_parameters(libs):
+    """Entry points that a program built on an earlier header calls: still exported, with the parameters they had (one
+    more in front of the stream would take the caller's stream for it without an error)."""
+    had = {"ng_query_index_dev": 13, "ng_act_next": 12, "ng_act_split": 11, "ng_scan_list_dev": 18,
+           "ng_scan_ids_emit": 16}
+    arity = declared_arity("ngram_amd.h")
+    assert {n: arity.get(n) for n in had} == had
+    assert all(hasattr(libs["ngram_amd.h"], n) for n in had)
+
+
 def test_engine_calls_match_the_header_arity():
     """Every call of an ng_* entry point through the ctypes wrapper (`lib("ng_x", ...)`, `lib.cub("ng_x", ...)` for
     the two-phase ones, `lib.size("ng_x", ...)` for the sizing ones) passes as many arguments as the prototype has,

@@ -89,3 +89,47 @@ def test_deep_levels_with_many_rounds_a_block(gpu, n_cand, grid, n_query, first)
         assert tuple(m[nlev, :2]) == trial
     if n_query == 2500 and n_cand == 20_000 and grid == 1:
         assert len(hits[K0 if not first else CAP]) > 4 * 4096  # several flushes of the stage
+
+
+@pytest.mark.parametrize("k", [3, 6])
+@pytest.mark.parametrize("n_dev", [0, 1, 700, 1900])
+def test_one_level_by_device_side_counts(gpu, k, n_dev):
+    """ng_query_index_dev, ng_scan_list_dev and ng_act_split over the first n_dev entries of their lists (their number
+    on the device): the contexts' hit bits, the hit positions, and the entries without a hit, against Python sets."""
+    rng = np.random.default_rng(10 * k + n_dev)
+    L, N, g = 32 * 200, 2000, 3
+    tok = rng.integers(0, 4, L).astype(np.uint16)
+    x = rng.integers(0, 4, N).astype(np.uint16)
+    avail = np.minimum(np.arange(N) + 1, rng.integers(1, 20, N)).astype(np.int32)
+    act = rng.permutation(N).astype(np.int32)[:1900]
+    cand = np.sort(rng.choice(L, 1900, replace=False)).astype(np.int64)
+    text, query = tok.astype(">u2").tobytes(), x.astype(">u2").tobytes()
+    ctx = {int(i): query[2 * (i - k + 1) : 2 * (i + 1)] for i in act[:n_dev] if avail[i] >= k}
+    hits = [int(p) for p in cand[:n_dev] if p >= k and text[2 * (p - k) : 2 * p] in set(ctx.values())]
+    seen = {text[2 * (p - k) : 2 * p] for p in hits}
+    done = {i for i, c in ctx.items() if c in seen}
+
+    lib, dev = Lib(), torch.device("cuda")
+    put = lambda a: torch.from_numpy(a).to(dev)  # noqa: E731
+    slots, qcap = 8192, 7168
+    d_tok, d_x, d_act, d_cand = put(tok.view(np.int16)), put(x.view(np.int16)), put(act), put(cand)
+    d_n = torch.tensor([n_dev], dtype=torch.int64, device=dev)
+    table = torch.empty(slots, dtype=torch.int64, device=dev)
+    rep, hit = torch.empty(slots, dtype=torch.int32, device=dev), torch.zeros(slots // 32, dtype=torch.int32, device=dev)
+    ctx_of, out = (torch.full((1900,), -7, dtype=torch.int32, device=dev) for _ in range(2))
+    length, flags = torch.zeros(N, dtype=torch.int32, device=dev), torch.zeros(2, dtype=torch.int32, device=dev)
+    counters, n_out, matched = (torch.zeros(3, dtype=torch.int64, device=dev) for _ in range(3))
+    lib("ng_query_index_dev", d_x, put(avail), d_act, d_n, 1900, i32(k), table, u64(qcap), u64(slots), rep, ctx_of,
+        counters)
+    R = 768  # 3 blocks, 256 positions a round
+    ev, ev_count = torch.empty(g * R, dtype=torch.int64, device=dev), torch.zeros(g, dtype=torch.int32, device=dev)
+    lib("ng_scan_list_dev", d_tok, i32(k), d_cand, d_n, 1900, table, u64(qcap), rep, d_x, hit, i32(1), ev, u64(R), ev_count,
+        flags, i32(g), u64(0))
+    lib("ng_act_split", d_act, d_n, 1900, ctx_of, hit, i32(k), length, out, n_out, matched)
+    assert not counters[1:].any() and not flags.any()
+    assert (ctx_of[n_dev:] == -7).all()
+    got = np.concatenate([ev[b * R : b * R + int(c)].cpu().numpy() for b, c in enumerate(ev_count.tolist())])
+    assert sorted(got.tolist()) == hits
+    assert set(np.flatnonzero(length.cpu().numpy())) == done and int(matched[0]) == len(done)
+    left = out[: int(n_out[0])].tolist()
+    assert sorted(left) == sorted(set(act[:n_dev].tolist()) - done)
