@@ -446,6 +446,8 @@ class OnlineRows:
         without its launches and merges per step."""
         taus, step_lo, step_hi = self._rule(rule, step_lo, step_hi)
         cfg = self._check_config((), (1,), 0, count_levels)
+        if not cfg[3]:
+            raise ValueError("need count levels")
         tau, tau_in, last = taus if taus is not None else (self.tau, self.tau_in, self.max_step)
         n, dev, lib = self.n, self.dev, self.lib
         outs = self._device_outputs(cfg)
@@ -457,6 +459,8 @@ class OnlineRows:
             qa, qb = self._range(steps, step_lo, step_hi)
             rows = qpos = order[qa:qb]
             mq = qb - qa
+        if mq == 0:
+            return outs, rows
         nc = len(count_levels)
         bits = max(1, (last + 2).bit_length())
         none = (1 << bits) - 1

@@ -30,3 +30,21 @@ def test_counts_match_the_stepwise_state(gpu, n, parts, vocab, rule, lo, hi):
         assert torch.equal(got[name], want[name]), name
     if n >= 6000 and (lo, hi) in ((0, 12), (0, 0)):  # the streams' draws leave counted contexts to compare
         assert int(got["tot"].max()) > 3
+
+
+def test_calls_at_the_edge_of_what_is_taken(gpu):
+    """No levels raise ValueError; a level past the kernels' longest context raises once a query is asked of it, and a
+    range without queries asks none."""
+    n = 1000
+    tok = np.random.default_rng(0).integers(0, 5, n).astype(np.uint16)
+    rows = OnlineRows(tok, [0, n], [(0, 500, 2), (500, n, 5)])
+    with pytest.raises(ValueError):
+        rows.segment_counts([])
+    with pytest.raises(RuntimeError):
+        rows.segment_counts([65])
+    out = [np.full((n, 1), 7, t) for t in (np.uint32, np.uint16, np.uint32)]
+    with pytest.raises(RuntimeError):
+        rows.counts([65], 0, 6, *out)
+    for lo, hi in ((0, 0), (0, 2), (3, 5), (6, 9)):
+        rows.counts([65], lo, hi, *out)
+    assert all((o == 7).all() for o in out)
