@@ -5,6 +5,7 @@ out-of-order spans, parts and end-of-text tokens, contexts longer than a part, s
 import numpy as np
 import pytest
 
+from ngram_amd import online
 from ngram_amd.online import NONE, OnlineRows
 
 pytestmark = pytest.mark.gpu
@@ -52,3 +53,26 @@ def test_training_order(gpu, n, parts, spread):
         assert np.array_equal(order.cpu().numpy(), want), k
         for s in {0, 1, int(spread), int(spans[:, 2].max()) + 1, *step[want].tolist()}:
             assert steps.before(int(s)) == int((step[want] < s).sum()), (k, s)
+
+
+@pytest.mark.parametrize("m,top", [(40, 40), (40, 1100), (40, 1200), (40, 1_000_000), (3000, 7000), (3000, 7100)])
+def test_bounds_of_steps_close_together_and_apart(gpu, m, top, monkeypatch):
+    """A few spans whose steps are far apart keep bounds of the steps in use, not of every step up to the last (host
+    arrays of a million entries per level otherwise); both forms give the same bounds and the same largest step."""
+    rng = np.random.default_rng(m)
+    n = 8000
+    at = np.linspace(0, n, m + 1).astype(np.int64)
+    steps = np.append(np.sort(rng.choice(top - 1, m - 1, replace=False)), top - 1)
+    spans = np.stack([at[:-1], at[1:], rng.permutation(steps)], 1)
+    tok = rng.integers(0, 9, n).astype(np.uint16)
+    got = {}
+    for table in (online.STEP_TABLE, 0):
+        monkeypatch.setattr(online, "STEP_TABLE", table)
+        rows = OnlineRows(tok, [0, n], spans)
+        got[table] = rows._by_step([(rows.tau_in, 0), (rows.tau, 2)], rows.max_step + 1)
+    for (o1, b1), (o2, b2) in zip(*got.values()):
+        assert np.array_equal(o1.cpu().numpy(), o2.cpu().numpy())
+        assert len(b1.steps) <= 2 * m + 1026
+        for s in (0, 1, top // 2, top, *steps[:50].tolist()):
+            assert b1.before(int(s)) == b2.before(int(s)), s
+    assert rows._most([b for _, b in got[0]]) == rows._most([b for _, b in list(got.values())[0]])
