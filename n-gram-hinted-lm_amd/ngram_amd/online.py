@@ -40,6 +40,7 @@ def _i64_array(rows) -> ctypes.Array:
 
 NONE = 0xFFFFFFFF
 LOAD = 0.5
+MAX_LEVEL = 64  # tokens of the longest context the kernels take
 
 
 def loader_plan(ntok, nproc: int, BT: int, accum: int, steps: int) -> np.ndarray:
@@ -98,6 +99,11 @@ def plan_rows(plan: np.ndarray, sizes: list[int], BT: int, accum: int, rank: int
 # itself. Looked up / listed, construction and prepare at four levels: 65536 positions, 1000 spans with steps below 1000
 # 0.84 / 1.00 ms, below 4000 0.99 / 0.90, below 64000 4.9 / 0.9; 2^20 positions, 65536 spans 5.7 / 6.0.
 STEP_TABLE = 1 << 20
+# A stream of at least FEW_MIN positions of which fewer than one in FEW_SHARE are trained has its trained positions picked
+# out before they are sorted, so that sorts, tables and kept lists are as long as they are, not as the stream is.
+# Of 2^26 positions, all sorted / the trained ones: half trained, order 4.6 / 6.1 ms and counts of three levels 57 / 46; a
+# quarter 4.6 / 4.9 and 42 / 24; 1 in 64 4.6 / 3.7 and 31 / 5.9, the prepared state 1552 / 544 MiB.
+FEW_MIN, FEW_SHARE = 1 << 20, 4
 
 
 class _Steps:
@@ -152,6 +158,7 @@ class OnlineRows:
                  self.tau_in)
         self.max_step = int(sp[:, 2].max()) if len(sp) else -1
         self.max_steps = len(sp)  # at most this many steps are in use
+        self._trained = None  # how many positions have a step, once asked for
         seg = torch.empty(n, dtype=torch.int64, device=dev)
         self.has_next = torch.empty(n, dtype=torch.uint8, device=dev)
         self.lib("ng_online_layout", self.tok, n, self.bounds_dev, np_, seg, self.has_next)
@@ -268,22 +275,38 @@ class OnlineRows:
             st["rows_desc"] = torch.tensor(desc, dtype=torch.int64, device=dev)
         return st
 
+    def _few(self, every: bool) -> bool:
+        """Whether few of the stream's positions have a step (every: all of them do, the rule "segment")."""
+        if every or self.n < FEW_MIN:
+            return False
+        if self._trained is None:
+            self._trained = int((self.tau != -1).sum().item())
+        return self._trained * FEW_SHARE < self.n
+
     def _by_step(self, lists: list, last: int, every: bool = False) -> list:
         """Per (tau, k) of `lists` the positions with a step, ordered by it and within a step by position (int32), and
-        the steps' bounds (ng_online_order's steps, at most `last`; a stable sort by them). every: every step is in use
-        (the rule "segment"'s are)."""
+        the steps' bounds (ng_online_order's steps, at most `last`; a stable sort by them). every: every position has a
+        step, and every step is in use (the rule "segment")."""
         n, dev = self.n, self.dev
         bits = max(1, (last + 1).bit_length())
         none = (1 << bits) - 1  # above every step: the positions without one sort behind the others
         table = last < STEP_TABLE and (every or last <= 2 * self.max_steps + 1024)
         steps = torch.arange(last + 2, device=dev) if table else None
-        key, key2 = (torch.empty(n, dtype=torch.int64, device=dev) for _ in range(2))
+        few = self._few(every)
+        key = torch.empty(n, dtype=torch.int64, device=dev)
         val = torch.empty(n, dtype=torch.int32, device=dev)
+        key2 = None if few else torch.empty(n, dtype=torch.int64, device=dev)
         out, bounds = [], []
         for tau, k in lists:
-            order = torch.empty(n, dtype=torch.int32, device=dev)
             self.lib("ng_online_order", tau, n, self.bounds_dev, len(self.bounds) - 1, i32(k), u64(none), key, val)
-            self.lib.cub("sort_pairs", key, key2, val, order, n, i32(0), i32(bits))
+            m, key1, val1 = n, key, val
+            if few:
+                val1 = torch.nonzero(key != none).squeeze(1)
+                m, key1, val1 = val1.numel(), key[val1], val1.to(torch.int32)
+                key2 = torch.empty(m, dtype=torch.int64, device=dev)
+            order = torch.empty(m, dtype=torch.int32, device=dev)
+            if m:
+                self.lib.cub("sort_pairs", key1, key2, val1, order, m, i32(0), i32(bits))
             out.append(order)
             if table:
                 bounds.append(torch.searchsorted(key2, steps))
@@ -292,7 +315,7 @@ class OnlineRows:
                 u, c = u.cpu().numpy(), c.cpu().numpy()
                 begins = np.cumsum(c) - c
                 at = int(np.searchsorted(u, none))
-                bounds.append(_Steps(u[:at], begins[:at], int(begins[at]) if at < len(u) else n))
+                bounds.append(_Steps(u[:at], begins[:at], int(begins[at]) if at < len(u) else m))
         if table:
             host = torch.stack(bounds).cpu().numpy()  # one read for every list
             bounds = [_Steps(np.arange(last + 1), h[:-1], int(h[-1])) for h in host]
@@ -468,29 +491,42 @@ class OnlineRows:
         if mq == 0:
             return outs, rows
         nc = len(count_levels)
+        if max(count_levels) > MAX_LEVEL:
+            raise RuntimeError(f"k={max(count_levels)}: a context has at most {MAX_LEVEL} tokens")
         bits = max(1, (last + 2).bit_length())
         none = (1 << bits) - 1
-        cap = max(1 << 16, int(n / LOAD) + 1)
+        few = self._few(rule == "segment")
+        most = max(1, self._trained) if few else n  # a level's occurrences end at trained positions
+        cap = max(1 << 16, int(most / LOAD) + 1)
         cbits = cap.bit_length()
-        u64s = [torch.empty(n, dtype=torch.int64, device=dev) for _ in range(4)]
-        u32s = [torch.empty(n, dtype=torch.int32, device=dev) for _ in range(4)]
+        u64s = [torch.empty(most, dtype=torch.int64, device=dev) for _ in range(4)]
+        u32s = [torch.empty(most, dtype=torch.int32, device=dev) for _ in range(4)]
+        # the steps of the whole stream, of which the occurrences are picked out where they are few
+        order = (torch.empty(n, dtype=torch.int64, device=dev), torch.empty(n, dtype=torch.int32, device=dev)) \
+            if few else (u64s[0], u32s[0])
         ck = torch.empty(cap, dtype=torch.int64, device=dev)
         bounds = torch.empty((cap, 2), dtype=torch.int32, device=dev)
-        first = torch.empty(n, dtype=torch.uint8, device=dev)
-        pre = torch.empty(n + 1, dtype=torch.int32, device=dev)
+        first = torch.empty(most, dtype=torch.uint8, device=dev)
+        pre = torch.empty(most + 1, dtype=torch.int32, device=dev)
         flags = torch.zeros((len(set(count_levels)), 2), dtype=torch.int32, device=dev)
         ks = sorted(set(count_levels))
         for k, flag in zip(ks, flags):
             (key, ka, kb, akey), (val, va, vb, occ) = u64s, u32s
-            lib("ng_online_order", tau, n, self.bounds_dev, len(self.bounds) - 1, i32(k), u64(none), key, val)
-            lib.cub("sort_pairs", key, akey, val, occ, n, i32(0), i32(bits))
+            lib("ng_online_order", tau, n, self.bounds_dev, len(self.bounds) - 1, i32(k), u64(none), *order)
+            m, step_of, at = n, *order
+            if few:
+                at = torch.nonzero(step_of != none).squeeze(1)
+                m, step_of, at = at.numel(), step_of[at], at.to(torch.int32)
+            if m == 0:
+                continue
+            lib.cub("sort_pairs", step_of, akey, at, occ, m, i32(0), i32(bits))
             lib.fill(ck, -1)
-            lib("ng_online_occ_insert", self.tok, occ, akey, u64(none), n, i32(k), ck, u64(cap), i32(cbits), key, val,
+            lib("ng_online_occ_insert", self.tok, occ, akey, u64(none), m, i32(k), ck, u64(cap), i32(cbits), key, val,
                 flag)
-            lib.cub("sort_pairs", key, ka, val, va, n, i32(0), i32(16 + cbits))
-            lib.cub("sort_pairs", key, kb, val, vb, n, i32(16), i32(16 + cbits))
-            lib.cub("ng_online_occ_index", ka, va, kb, vb, n, i32(cbits), first, pre, bounds)
-            lib("ng_online_occ_query", self.tok, self.avail, self.has_next, qpos, mq, tau_in, akey, n, i32(k), ck,
+            lib.cub("sort_pairs", key, ka, val, va, m, i32(0), i32(16 + cbits))
+            lib.cub("sort_pairs", key, kb, val, vb, m, i32(16), i32(16 + cbits))
+            lib.cub("ng_online_occ_index", ka, va, kb, vb, m, i32(cbits), first, pre, bounds)
+            lib("ng_online_occ_query", self.tok, self.avail, self.has_next, qpos, mq, tau_in, akey, m, i32(k), ck,
                 u64(cap), bounds, vb, pre, ka, va, outs["tot"], outs["dist"], outs["cnt"], i32(nc),
                 i32(count_levels.index(k)))
         for k, f in zip(ks, flags[:, 0].cpu().tolist()):

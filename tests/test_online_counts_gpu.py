@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 import torch
 
+from ngram_amd import online
 from ngram_amd.online import OnlineRows
 
 pytestmark = pytest.mark.gpu
@@ -48,3 +49,31 @@ def test_calls_at_the_edge_of_what_is_taken(gpu):
     for lo, hi in ((0, 0), (0, 2), (3, 5), (6, 9)):
         rows.counts([65], lo, hi, *out)
     assert all((o == 7).all() for o in out)
+
+
+@pytest.mark.parametrize("trained", [0, 1, 2, 300, 4800])
+@pytest.mark.parametrize("spread", [1, 3_000_000])
+def test_a_stream_of_which_few_positions_are_trained(gpu, trained, spread, monkeypatch):
+    """Picking the trained positions out before they are sorted gives the state and the count rows that sorting the whole
+    stream gives, and keeps lists only as long as they are."""
+    n, m = 20_000, max(1, trained // 40)
+    rng = np.random.default_rng(trained)
+    tok = rng.integers(0, 6, n).astype(np.uint16)
+    tok[rng.random(n) < 0.01] = 50256
+    at = rng.choice(n // 50 - 1, m, replace=False) * 50
+    size = np.full(m, 40) if trained >= 40 else np.full(m, trained)
+    spans = np.stack([at, at + size, rng.integers(0, 7, m) * spread], 1)
+    got = {}
+    for few in (1, 1 << 40):
+        monkeypatch.setattr(online, "FEW_MIN", few)
+        rows = OnlineRows(tok, [0, n // 3, n], spans)
+        rows.prepare([1, 3], [1, 3], 4, [1, 3, 9])
+        lists = [rows.state["q_pos"]] + [lv["occ"] for lv in rows.state["levels"].values()]
+        out = [np.zeros((n, 3), t) for t in (np.uint32, np.uint16, np.uint32)]
+        rows.counts([3, 1, 9], 0, 7 * spread, *out)
+        got[few] = [t.cpu().numpy() for t in lists] + out
+        if few == 1:
+            assert all(t.untyped_storage().nbytes() <= 4 * t.numel() for t in lists)
+    for a, b in zip(*got.values()):
+        assert np.array_equal(a, b)
+    assert trained < 300 or got[1][-3].max() > 1
