@@ -175,7 +175,10 @@ __global__ void __launch_bounds__(1024) batch_scan_k(u32* __restrict__ work, i64
 // block sums those before its tile and all of them itself (at most BR_RAW_TILES: a few loads a thread, from L2), block 0
 // stores *total and every block pads its share. Two launches instead of four for a training batch, whose time is its
 // launches: 65536 positions, 39.1 us a call with four and the total copied back, 30.5 with two and the total written to
-// host memory. Past BR_RAW_TILES every block's sums would cost more than the scan's launch.
+// host memory. Past BR_RAW_TILES every block's sums would cost more than the scan's launch; and a capacity past every
+// entry of the tiles' positions (8 each) is padding for the few tiles' blocks alone, where the padding kernel takes as
+// many as the capacity fills: one tile with room for 8192, 16384, 32768 and 262144 entries, 21.7, 24.3, 30.0 and 105 us
+// here, 24 us each in four launches (64 tiles with that room each: 23.5, 26.5, 32.8 and 108; 25.9, 26.7, 28.4 and 47).
 #define BR_RAW_TILES 1024
 template <bool RAW>
 __global__ void __launch_bounds__(256) batch_write_k(const int* __restrict__ cells, const int* __restrict__ entries,
@@ -286,7 +289,7 @@ static int launch_batch_rows(const int* cells, const int* entries, i64 n, i64 ca
                              u64* total, hipStream_t st) {
     const i64 tiles = (n + BR_TILE - 1) / BR_TILE;
     batch_count_k<<<(int)tiles, 256, 0, st>>>(entries, n, work);
-    if (tiles <= BR_RAW_TILES) {
+    if (tiles <= BR_RAW_TILES && capacity <= tiles * BR_TILE * 8) {
         batch_write_k<true><<<(int)tiles, 256, 0, st>>>(cells, entries, n, capacity, work, tiles, total, out);
         return (int)hipGetLastError();
     }

@@ -90,6 +90,26 @@ def test_batch_rows_many_tiles(gpu):
     assert np.array_equal(out.cpu().numpy(), O.batch_rows(cells, entries, 0, n, cap))
 
 
+@pytest.mark.parametrize("n", [1, 1023, 1024, 1025, 2500])
+@pytest.mark.parametrize("over", [-1, 0, 1, 300_000])
+@pytest.mark.parametrize("pinned", [True, False])
+def test_batch_rows_around_the_room_of_its_tiles(gpu, n, over, pinned):
+    """Capacities below, at and far past every entry of the tiles' positions (padded by the writing blocks, or by a kernel
+    of its own), the total in host or device memory."""
+    lib = Lib()
+    rng = np.random.default_rng(n)
+    cells = rng.integers(0, 99, n).astype(np.int32)
+    entries = np.where(rng.random((n, 8)) < 0.4, rng.integers(1, 1 << 20, (n, 8)), 0).astype(np.int32)
+    cap = -(-n // 1024) * 8192 + over
+    out = torch.empty(n + 2 * cap, dtype=torch.int32, device="cuda")
+    work = torch.empty(lib.size("ng_batch_rows_work", n), dtype=torch.int32, device="cuda")
+    total = torch.zeros(1, dtype=torch.int64, pin_memory=True) if pinned else \
+        torch.zeros(1, dtype=torch.int64, device="cuda")
+    lib("ng_batch_rows", torch.from_numpy(cells).cuda(), torch.from_numpy(entries).cuda(), n, cap, out, work, total)
+    assert np.array_equal(out.cpu().numpy(), O.batch_rows(cells, entries, 0, n, cap))
+    assert int(total.item()) == int((entries != 0).sum())
+
+
 def test_batch_rows_refuses_positions_past_its_offsets(gpu):
     """The tiles' offsets and the running offset are u32 (8 entries per position): n above (2^32 - 1) / 8 is refused
     before any launch (the buffers here are far smaller than such an n: nothing may be read)."""
