@@ -189,7 +189,13 @@ class LevelBuild:
             use32 = W <= W_MAX and k not in self.wide and \
                 (cnt_top is None or (self.level_shards[k] > 0 and n_reg < 1 << 32))
             if not use32 and seen_n is not None:  # the 64-bit count takes an exact list: read its length
-                seen = seen[: int(seen_n.item())]
+                n_seen = int(seen_n.item())
+                if n_seen > seen_cap:  # more than their room, so the index holds a cut list: run again with room for them
+                    self.seen_of[k] = n_seen
+                    self.reruns += 1
+                    return self.build(x, tgt, avail, topk=topk, cnt_top=cnt_top, keep=keep, with_mask=with_mask,
+                                      stats=want_stats, _defer=_defer)
+                seen = seen[:n_seen]
                 seen_n = None
             if not use32 and cnt_top is not None:
                 ktop = 8  # its thresholds find a context's words by its record's first word, which top 8 has room for

@@ -47,3 +47,25 @@ def test_top_rule_matches_oracle(corpus, cnt_top, mode, monkeypatch):
         assert np.array_equal(res.mask.cpu().numpy(), mask)
     assert set(res.kept) == {2, 8}
     assert (out[1, 1] > 4).any() and (mode == "64-bit" or not eng.wide)
+
+
+@pytest.mark.parametrize("cnt_top", [None, 4])
+def test_position_list_that_outgrows_its_room_on_the_64_bit_count(corpus, cnt_top, monkeypatch):
+    """A later build whose levels have far more positions with an occurred context than the last one's, but no more
+    contexts: the positions listed on the device outrun their room, which the 64-bit count has to notice too."""
+    monkeypatch.setattr(levels_mod, "W_MAX", 0)
+    tok, sizes, starts, _ = data.device_tokens(corpus.shards())
+    eng = levels_mod.LevelBuild(tok, sizes, starts, LEVELS)
+    block = corpus.train[1000:9000]
+    absent = np.setdiff1d(np.arange(50000), corpus.train)[0]
+    for q in (np.append(block, np.full(24_000, absent, np.uint16)), np.tile(block, 4)):
+        q = q.astype(np.uint16)
+        x, tgt, avail = C.queries(q, [], "cuda")
+        out = eng.build(x, tgt, avail, cnt_top=cnt_top).counts.cpu().numpy()
+        for li, k in enumerate(LEVELS):
+            o = O.query_counts(corpus.train, corpus.bounds, q[:-1], q[1:], O.segments(q[:-1]), k,
+                               cnt_top=cnt_top or 1 << 30)
+            assert np.array_equal(out[0, li].view(np.uint32), o["tot"]), f"tot k={k}"
+            assert np.array_equal(out[1, li], o["dist"].astype(np.int32)), f"dist k={k}"
+            assert np.array_equal(out[2, li].view(np.uint32), o["cnt"]), f"cnt k={k}"
+    assert eng.reruns > 0
