@@ -26,6 +26,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 
 import numpy as np
 import torch
@@ -111,7 +112,7 @@ class CountTable:
         self.tables: list[_Level] = []
         self.built = self.released = False
         self.grid = torch.cuda.get_device_properties(dev).multi_processor_count * EMIT_BLOCKS_PER_CU
-        self.events: list = []
+        self._events: list = []
         torch.cuda.synchronize(dev)
         return self
 
@@ -133,7 +134,7 @@ class CountTable:
         self._tokens = int(sum(sizes))
         self.tables, self.built, self.released = [], False, False
         self.grid = torch.cuda.get_device_properties(tok.device).multi_processor_count * EMIT_BLOCKS_PER_CU
-        self.events = []
+        self._events = []
         return self
 
     @property
@@ -162,12 +163,25 @@ class CountTable:
         for k in self._levels:
             self.tables.append(self._build_level(k))
 
+    @property
+    def events(self) -> list:
+        """The launches so far with their timing events: (name, k, start, end). Builds and queries record them where `timed`
+        was set before them; a built table that recorded none gives an empty list, with a warning."""
+        if self.built and not self.timed:
+            warnings.warn("the table recorded no events: set timed = True on it before the build", RuntimeWarning,
+                          stacklevel=2)
+        return self._events
+
+    @events.setter
+    def events(self, events: list) -> None:
+        self._events = events
+
     def _timed(self, name: str, k: int):
         """Timing events around a launch, kept in `events`, where the table is `timed`."""
         if not self.timed:
             return P.NO_EVENTS
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        self.events.append((name, k, e0, e1))
+        self._events.append((name, k, e0, e1))
         return e0, e1
 
     def _build_level(self, k: int) -> _Level:

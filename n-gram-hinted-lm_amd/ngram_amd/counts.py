@@ -100,7 +100,8 @@ class CountBuild:
 
     @property
     def kernel_events(self) -> list:
-        """The last build's launches with their timing events (LevelBuild._event), if `engine.timed` was set before it."""
+        """The last build's launches with their timing events (LevelBuild.kernel_events: recorded where `engine.timed` was
+        set before it)."""
         return self.engine.kernel_events
 
     def prepare(self) -> None:

@@ -27,6 +27,7 @@ next build of the same inputs."""
 from __future__ import annotations
 
 import time
+import warnings
 from dataclasses import dataclass, field
 
 import torch
@@ -86,8 +87,9 @@ class LevelBuild:
         self.events_of: dict[int, int] = {}
         self.contexts_of: dict[int, int] = {}
         self.dratio: dict[int, float] = {}
-        self.kernel_events: list = []
+        self._events: list = []
         self.timed = False  # whether builds record kernel_events
+        self._untimed = False  # whether the last build recorded none
         self.host_s = {"index": 0.0, "scan": 0.0, "count": 0.0}
         self._plist = None
         self._no_bm = None  # the level whose list scan sets no hit bits (the last one, without hit statistics)
@@ -95,6 +97,15 @@ class LevelBuild:
         self.min_pbits: dict[int, int] = {}  # per level, partition bits the 32-bit count found too few, plus one
         self.seen_of: dict[int, int] = {}  # per level, the query positions whose previous level's context occurred
         self.reruns = 0  # builds run again (a size learnt from an earlier build fell short), over this engine's life
+
+    @property
+    def kernel_events(self) -> list:
+        """The last build's launches with their timing events (see _event). A build records them where `timed` was set
+        before it; after one that recorded none the list is empty, with a warning."""
+        if self._untimed:
+            warnings.warn("the last build recorded no kernel events: set timed = True on the engine before the build",
+                          RuntimeWarning, stacklevel=2)
+        return self._events
 
     def _event(self, name: str, k: int, n: int, mode: int = -1):
         """A pair of timing events around a launch on the current stream, kept in kernel_events as (name, k, n, e0,
@@ -104,7 +115,7 @@ class LevelBuild:
         if not self.timed:
             return partcount.NO_EVENTS
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        self.kernel_events.append((name, k, n, e0, e1, mode))
+        self._events.append((name, k, n, e0, e1, mode))
         return e0, e1
 
     def _wait(self, i: int) -> None:
@@ -119,7 +130,7 @@ class LevelBuild:
         `keep`: levels whose records are returned (top-8); `stats`: each level's corpus hits in info."""
         dev, N, elib = self.tok.device, x.numel(), self.elib
         want_stats = stats
-        self.kernel_events = []
+        self._events, self._untimed = [], not self.timed
         self.grid = torch.cuda.get_device_properties(dev).multi_processor_count * SCAN_BLOCKS_PER_CU
         nwords = self.L // 32
         # the levels' hit bitmaps: a dense, sparse or compact scan writes every word of its range, so only a list
