@@ -41,7 +41,8 @@ from .qindex import LOAD as QLOAD, TAIL as QTAIL, QueryIndex
 
 
 _RATIO: dict[int, float] = {}  # distinct pairs per counted event at each level, from the last count (sizes partitions)
-_WIDE: set = set()  # levels whose 32-bit count overflowed its escape table: counted by the 64-bit path
+# levels (and "lists", the list levels together) whose 32-bit count overflowed by itself: counted by the 64-bit path
+_WIDE: set = set()
 # each existence level's query contexts per listed position in the last call: sizes the next call's query index for
 # its own number of positions
 _CONTEXTS: dict[int, float] = {}
@@ -215,12 +216,10 @@ def _count(elib: Lib, lib: Lib, tok, L: int, x, avail, levels: list, ladder: lis
                                                                                                     else []):
         if k == "lists":
             ids, ev = int(deep[2] / QLOAD) + 1024 + QTAIL, sum(levels[j - 1][2] for j in lists)
-            wide = lists[0] in _WIDE
         else:
             ids, ev = levels[k - 1][6], grid * R
-            wide = k in _WIDE
         ids = (ids + 31) // 32 * 32  # each level's final bits start at a word
-        if wide or w_bits(ids)[1] > W_MAX:  # by the 64-bit count, alone
+        if k in _WIDE or w_bits(ids)[1] > W_MAX:  # by the 64-bit count, alone
             _count_wide(elib, lib, tok, L, x, avail, [k], lists, levels, length, flags, grid, nxt, cnt)
             continue
         if group and (w_bits(used + ids)[1] > W_MAX or cap_ev + ev > GROUP_EVENTS):
@@ -315,11 +314,15 @@ def _count_group(elib: Lib, lib: Lib, tok, L: int, x, avail, group: list, lists:
             min_pbits = c.pbits + 1
             continue
         break
-    if fl & 3:  # its escape table overflowed, or no more partition bits: these levels take the 64-bit count from now on
+    if fl & 3:  # its escape table overflowed, or no more partition bits
         del regions, seg, c, dhist
-        for k, _, _ in group:
-            _WIDE.add(lists[0] if k == "lists" else k)
-        _count_wide(elib, lib, tok, L, x, avail, [k for k, _, _ in group], lists, levels, length, flags, grid, nxt, cnt)
+        if len(group) > 1:  # one level's doing, or only all of them together: each by itself
+            for k, _, ids in group:
+                _count_group(elib, lib, tok, L, x, avail, [(k, 0, ids)], lists, levels, deep, length, flags, grid, nxt, cnt)
+            return
+        k = group[0][0]  # this level takes the 64-bit count from now on
+        _WIDE.add(k)
+        _count_wide(elib, lib, tok, L, x, avail, [k], lists, levels, length, flags, grid, nxt, cnt)
         return
     _RATIO[key] = n_u / max(1, n_ev)
     EVENTS[0] += n_ev

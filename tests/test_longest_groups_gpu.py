@@ -59,3 +59,38 @@ def test_longest_match_on_small_streams(gpu, n_train, n_query, vocab, cap, mask,
         for k, eligible, matched in ladder:
             assert matched == int((want[0] >= k).sum()) and eligible == int((asked & (avail >= k)).sum())
         assert len(ladder) >= int(want[0].max())
+
+
+@pytest.mark.parametrize("overflows", [(1,), (3,), ("lists",), (2, "lists"), "together"])
+def test_a_group_that_overflows_marks_only_the_levels_that_do(gpu, overflows, monkeypatch):
+    """Levels counted together whose count reports a full escape table (forced here on counts that hold a given level, or
+    on counts of several levels): each is counted again by itself, and only one that overflows alone takes the 64-bit
+    count from then on."""
+    monkeypatch.setattr(LG, "_WIDE", set())
+    groups, count_group, count32 = [], LG._count_group, LG.count32
+
+    def grouped(*args):
+        groups.append([k for k, _, _ in args[6]])
+        return count_group(*args)
+
+    def counted(*args, **kw):
+        c = count32(*args, **kw)
+        if len(groups[-1]) > 1 if overflows == "together" else set(overflows) & set(groups[-1]):
+            c.stat[2] = 2
+        return c
+
+    monkeypatch.setattr(LG, "_count_group", grouped)
+    monkeypatch.setattr(LG, "count32", counted)
+    train, bounds, x = _streams(30000, 4097, 300, 11)
+    tok, _, _, _ = device_tokens([train[a:b] for a, b in zip(bounds, bounds[1:])])
+    xt = torch.from_numpy(x.view(np.int16)).cuda()
+    want = O.longest_match(train, bounds, x, O.segments(x), 64)
+    for _ in range(2):
+        length, nxt, cnt, _ = LG.longest_match(tok, xt, LG._segments(xt, Lib()), 64)
+        assert np.array_equal(length.cpu().numpy().view(np.uint32), want[0])
+        assert np.array_equal(nxt.cpu().numpy().view(np.uint16), want[1])
+        assert np.array_equal(cnt.cpu().numpy().view(np.uint32), want[2])
+    ks = {k for g in groups for k in g}
+    assert "lists" in ks and len(ks) > 2 and len(groups[0]) > 1
+    assert LG._WIDE == (set() if overflows == "together" else set(overflows) & ks)
+    assert LG._WIDE or overflows == "together"
