@@ -219,7 +219,9 @@ def _count(elib: Lib, lib: Lib, tok, L: int, x, avail, levels: list, ladder: lis
         else:
             ids, ev = levels[k - 1][6], grid * R
         ids = (ids + 31) // 32 * 32  # each level's final bits start at a word
-        if k in _WIDE or w_bits(ids)[1] > W_MAX:  # by the 64-bit count, alone
+        # by the 64-bit count, alone: a level that needs it, and list levels of more positions than one of its batches takes
+        # (room for all of them at once is 8 bytes each several times over, and the 32-bit count's offsets end at 2^32)
+        if k in _WIDE or w_bits(ids)[1] > W_MAX or (k == "lists" and ev > BATCH_EVENTS):
             _count_wide(elib, lib, tok, L, x, avail, [k], lists, levels, length, flags, grid, nxt, cnt)
             continue
         if group and (w_bits(used + ids)[1] > W_MAX or cap_ev + ev > GROUP_EVENTS):
@@ -356,7 +358,7 @@ EVENTS = [0]  # (context, next) events the last longest_match counted (its count
 DEVICE_LEVELS = True  # the existence phase's levels after the second list level run without host syncs
 LONG_FIRST = 8  # the device levels try level cap first when at least this many levels lie between
 GROUP_EVENTS = 1 << 26  # bitmap levels counted together until their scan regions hold this many events
-BATCH_EVENTS = 1 << 28  # list levels counted together until their listed positions reach this
+BATCH_EVENTS = 1 << 28  # list levels counted together by the 64-bit count until their listed positions reach this
 LIST_DIV = 64  # a level's hits go to a position list once fewer than L / LIST_DIV (8 B each against L / 8 bitmap bytes)
 
 

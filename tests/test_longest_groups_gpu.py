@@ -94,3 +94,35 @@ def test_a_group_that_overflows_marks_only_the_levels_that_do(gpu, overflows, mo
     assert "lists" in ks and len(ks) > 2 and len(groups[0]) > 1
     assert LG._WIDE == (set() if overflows == "together" else set(overflows) & ks)
     assert LG._WIDE or overflows == "together"
+
+
+def test_list_levels_past_one_batch_are_counted_in_batches(gpu, monkeypatch):
+    """List levels of more positions than a batch takes are not counted at once: their count's buffers would grow with
+    the number of levels, and past 2^32 positions its offsets would wrap."""
+    batches, count_batch, lists_emit = [], LG._count_batch, []
+
+    def batched(*args):
+        batches.append([args[7][k - 1][2] for k, _, _ in args[6]])
+        return count_batch(*args)
+
+    class Watched(Lib):
+        def __call__(self, name, *args):
+            if name == "ng_lm_lists_emit":
+                lists_emit.append(name)
+            return super().__call__(name, *args)
+
+    train, bounds, x = _streams(30000, 4097, 300, 12)
+    tok, _, _, _ = device_tokens([train[a:b] for a, b in zip(bounds, bounds[1:])])
+    xt = torch.from_numpy(x.view(np.int16)).cuda()
+    want = O.longest_match(train, bounds, x, O.segments(x), 64)
+    monkeypatch.setattr(LG, "_WIDE", set())
+    monkeypatch.setattr(LG, "_count_batch", batched)
+    for limit in (1 << 28, 200):
+        monkeypatch.setattr(LG, "BATCH_EVENTS", limit)
+        batches.clear(), lists_emit.clear()
+        length, nxt, cnt, _ = LG.longest_match(tok, xt, LG._segments(xt, Lib()), 64, elib=Watched())
+        assert np.array_equal(length.cpu().numpy().view(np.uint32), want[0])
+        assert np.array_equal(nxt.cpu().numpy().view(np.uint16), want[1])
+        assert np.array_equal(cnt.cpu().numpy().view(np.uint32), want[2])
+        assert (len(lists_emit), len(batches) > 1) == ((1, False) if limit > 200 else (0, True))
+    assert all(sum(b[:-1]) < 200 for b in batches) and sum(map(sum, batches)) > 200 and not LG._WIDE
