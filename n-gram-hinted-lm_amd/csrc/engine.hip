@@ -1689,8 +1689,8 @@ extern "C" int ng_act_split(const int* act, const u64* n_dev, i64 n_max, const i
 
 namespace {
 
-// The block's `mine` kept entries of each thread (4 at most) placed: the block's base (one atomic on *n_out) + the entries
-// of earlier threads. Every thread of a 256-thread block calls it.
+// The block's `mine` kept entries of each thread placed (any number of them; a block's sum in 32 bits): the block's base (one
+// atomic on *n_out) + the entries of earlier threads. Every thread of a 256-thread block calls it.
 __device__ __forceinline__ u64 place_in_block(u32 mine, u64* n_out, u32* s_wave, u64* s_base) {
     const int lane = lane_id(), w = threadIdx.x / WAVE;
     u32 incl = mine;
@@ -1770,8 +1770,9 @@ __global__ void __launch_bounds__(256) lm_tok1_k(const u16* __restrict__ x, cons
 }
 
 // A deep level's scan: the listed corpus positions whose k-context is in the table, appended to hl in no order, their
-// contexts marked lvl[id] = k. A block gathers its hits in LDS and takes their place with one atomic when LM_STAGE - 1024
-// of them are there or its entries end.
+// contexts marked lvl[id] = k. A block gathers its hits in LDS and takes their place with one atomic when more than
+// LM_STAGE - 1024 of them are there or its entries end (a list of at most 1024 positions a block, the longest match's
+// usual one, is one round).
 #define LM_STAGE 4096
 template <int K>
 __global__ void __launch_bounds__(256) lm_scan_k(const u16* __restrict__ tok, const u64* __restrict__ cand,

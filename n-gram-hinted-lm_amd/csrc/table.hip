@@ -408,7 +408,9 @@ extern "C" int ng_ctx_kth_grouped(const u64* w, const i64* gstart, int ibits, in
                                   u64* thr, void* stream) {
     if (kth < 1 || cb <= 0 || cb > 44 || esc_cap == 0 || gstart == nullptr || ibits < 0 || ibits > 11) return -1;
     if (m > 0) {
-        // with a device-side count, m only bounds it (by the pairs, far above the contexts that have kth of them)
+        // with a device-side count, m only bounds it (by the pairs, far above the contexts that have kth of them), and most
+        // of its blocks would find nothing: 100M tokens' validation statistics with at most 128, 512, 2048, 8192 and 65536
+        // blocks 18.16, 17.83, 17.80, 17.81 and 17.86 ms, 2M tokens' 4.19, 4.18, 4.19, 4.19 and 4.27
         const int most = m_dev ? 2048 : 65536;
         const int g = m < most ? (int)m : most;
         ctx_kth_k<<<g, 256, 0, (hipStream_t)stream>>>(w, cb, esc_k, esc_c, esc_cap, nullptr, ids, m, kth, thr, gstart,

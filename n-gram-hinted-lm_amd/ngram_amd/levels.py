@@ -361,7 +361,9 @@ class LevelBuild:
     def _load(self, k: int, prev, ktop: int, cnt_top) -> float | None:
         """Level k's query-table load: DENSE_LOAD where its scan probes every position (the first level, or behind a
         dense one) and a table at that load keeps the count's layout of one at the default load (the 32-bit count, its
-        runs mode: the same at both sizes, from the last build's context count); else None (the default)."""
+        runs mode: the same at both sizes, from the last build's context count); else None (the default). With a TOP
+        rule the default: more ids cost its count by words grouped by context what the scan gains (repeated builds of ten
+        levels over 100M tokens: 14.8 ms at the default, 14.9 at DENSE_LOAD)."""
         expect = self.contexts_of.get(k)
         if expect is None or (prev is not None and self._mode(1, [prev, k]) != 0):
             return None
@@ -370,8 +372,7 @@ class LevelBuild:
             ids = int(max(expect, 1) * max(EXPECT_MARGIN, 1.0) / load) + 1024 + QTAIL
             return w_bits(ids)[1] <= W_MAX, partcount.runs_fit(ids, ktop)
 
-        use32 = cnt_top is None and k not in self.wide
-        return DENSE_LOAD if use32 and layout(DENSE_LOAD) == layout(QLOAD) else None
+        return DENSE_LOAD if cnt_top is None and k not in self.wide and layout(DENSE_LOAD) == layout(QLOAD) else None
 
     @staticmethod
     def _mbits(W: int, ids: int, ktop: int) -> int:

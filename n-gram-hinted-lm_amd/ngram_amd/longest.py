@@ -357,7 +357,10 @@ TOK1_GRID = 2048  # level 1's scan blocks (each ORs its hit words into the level
 EVENTS = [0]  # (context, next) events the last longest_match counted (its counting phase), for its timing dict
 DEVICE_LEVELS = True  # the existence phase's levels after the second list level run without host syncs
 LONG_FIRST = 8  # the device levels try level cap first when at least this many levels lie between
-GROUP_EVENTS = 1 << 26  # bitmap levels counted together until their scan regions hold this many events
+# Levels are counted together until their scan regions hold this many events. At limits of 0 / 2^26 / 2^28 / 2^30: 4M tokens
+# 4.59 / 2.43 / 2.42 / 2.42 ms a call, 16M 9.17 / 6.85 / 6.59 / 6.59, 64M 15.8 / 15.8 / 13.8 / 13.5, 256M 31.7 / 31.8 / 31.8 /
+# 32.1, 1e9 115.4 at each; but a group's regions are held at once, and 64M tokens peak at 4.5 / 4.5 / 7.8 / 17.1 GiB.
+GROUP_EVENTS = 1 << 26
 BATCH_EVENTS = 1 << 28  # list levels counted together by the 64-bit count until their listed positions reach this
 LIST_DIV = 64  # a level's hits go to a position list once fewer than L / LIST_DIV (8 B each against L / 8 bitmap bytes)
 
