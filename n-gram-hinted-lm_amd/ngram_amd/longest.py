@@ -278,10 +278,6 @@ def _count_group(elib: Lib, lib: Lib, tok, L: int, x, avail, group: list, lists:
         table = elib.full_ones(slots, torch.int64, dev)
         rep = torch.empty(slots, dtype=torch.int32, device=dev)
         counters = elib.zeros((65, 3), torch.int64, dev)
-        mixed = SimpleNamespace(cap=qcap, ids=slots, table=table, rep=rep)
-        for k in lists:
-            QueryIndex(elib, x, avail, k, act0[:n0], compact=True, expect=n0, defer=True, counters=counters[k],
-                       shared=mixed)
         elib("ng_lm_index", x, act0, n0, length, i32(k0), table, u64(qcap), u64(slots), rep, i32(base), fid, counters)
         rows = (ctypes.c_int64 * (3 * len(lists)))(*[v for k in lists for v in (levels[k - 1][1].data_ptr(),
                                                                                levels[k - 1][2], k)])
@@ -504,19 +500,9 @@ def _count_batch(elib: Lib, lib: Lib, tok, L: int, x, avail, batch: list, levels
         elib("ng_seg_gather", regions, None, u64(R), None, ev_count, g, offs, ev, None)
         at = offs[g : g + 1].clone()
         del regions, ev_count
-    pending = [(k, vi.pending) for k, _, vi in batch if vi.n is None]  # deferred indexes' counters
-    got = torch.cat([at, flags[:1].to(torch.int64)] + [c for _, c in pending]).tolist()  # one copy
-    n_ev, fl = got[:2]
+    n_ev, fl = torch.cat([at, flags[:1].to(torch.int64)]).tolist()  # one copy
     if fl & 4:
         raise RuntimeError(f"levels {batch[0][0]}..{batch[-1][0]}: an emit region overflowed")
-    for j, (k, _) in enumerate(pending):
-        _, over, coll = got[2 + 3 * j : 5 + 3 * j]
-        if coll:
-            raise RuntimeError(f"k={k}: {coll} query positions collide with another context's key")
-        if over:  # an insert found no slot (a walk past its bound): the batch again, its indexes checked
-            del ev
-            redo = [(k2, f, QueryIndex(elib, x, avail, k2, f, compact=True)) for k2, f, _ in batch]
-            return _count_batch(elib, lib, tok, L, x, avail, redo, levels, flags, grid, nxt, cnt)
     key = ("batch", batch[0][0])
     c = count_events(elib, lib, ev, n_ev, n_ids, _RATIO.get(key, 1.0), presort="ctx")
     del ev

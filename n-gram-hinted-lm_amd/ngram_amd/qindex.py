@@ -22,8 +22,7 @@ EXPECT_MARGIN = 1.2  # a table sized from an expected context count holds this m
 class QueryIndex:
     def __init__(self, lib: Lib, x: torch.Tensor, avail: torch.Tensor, k: int, positions: torch.Tensor | None = None,
                  compact: bool = False, expect: int | None = None, _resized: bool = False, defer: bool = False,
-                 n_dev: torch.Tensor | None = None, counters: torch.Tensor | None = None, load: float | None = None,
-                 shared: "QueryIndex | None" = None):
+                 n_dev: torch.Tensor | None = None, counters: torch.Tensor | None = None, load: float | None = None):
         """Index the valid k-contexts of the query positions (all of x, or the int32 `positions`). `compact`: ctx_of
         holds one entry per listed position (in their order) instead of one per position of x. `expect`: about how
         many contexts there are (e.g. the last build's count): the table is sized for them at once instead of for
@@ -36,13 +35,7 @@ class QueryIndex:
         read; `positions` holds at least that many, or the caller checks). `counters` (int64 [3] of zeros on the device,
         with `defer`): where the deferred build's counters go (e.g. a row of the caller's stats, read with its other
         results in one copy), else new. `load`: the contexts per slot a table sized from a context count aims at (LOAD
-        if None); a sparser table shortens the probe walks of a level probed at every position. `shared` (with `defer` and
-        `counters`): this level's contexts go into another index's table, filled by its owner for several levels at once;
-        here only the level's counters are held."""
-        if shared is not None:
-            self.pending, self.n, self._valid = counters, None, None
-            self.cap, self.ids, self.table, self.rep = shared.cap, shared.ids, shared.table, shared.rep
-            return
+        if None); a sparser table shortens the probe walks of a level probed at every position."""
         dev = x.device
         ld = LOAD if load is None else load
         N = x.numel()

@@ -93,9 +93,10 @@ def test_device_levels_match_host_levels(corpus, monkeypatch):
 
 
 def test_unchecked_index_that_overflowed_counts_its_batch_again(corpus, monkeypatch):
-    """The list levels' query indexes are built without a host wait and checked once, with their batch's event
-    total. One that reports an insert without a slot (forced here from the host, on an index that is in fact whole)
-    makes the batch count again on indexes checked as they are built: the same outputs."""
+    """The list levels' final contexts share one table, filled without a host wait and checked once, with their count's
+    event total. One that ran out of slots (forced here by a table of 7 slots for some of its contexts, all of whose
+    inserts are refused but for a few, or all of them) makes the list levels count again on indexes checked as they are
+    built: the same outputs."""
     from ngram_amd import longest as LG
 
     x = corpus.query[:-1]
@@ -103,20 +104,31 @@ def test_unchecked_index_that_overflowed_counts_its_batch_again(corpus, monkeypa
     xt = torch.from_numpy(x.view(np.int16).copy()).cuda()
     av = _segments(xt, Lib())
     want = longest_match(tok, xt, av, 64)
-    flagged = []
+    again, count_wide = [], LG._count_wide
 
-    class Flagged(LG.QueryIndex):
-        def __init__(self, *a, **kw):
-            super().__init__(*a, **kw)
-            if kw.get("defer") and self.n is None:
-                self.pending[1] = 1
-                flagged.append(a[3])
+    def wide(*args):
+        again.append(args[6])
+        return count_wide(*args)
 
-    monkeypatch.setattr(LG, "QueryIndex", Flagged)
-    got = longest_match(tok, xt, av, 64)
-    assert len(flagged) > 10
-    for g, w in zip(got[:3], want[:3]):
-        assert torch.equal(g, w)
+    class Small(Lib):
+        def __call__(self, name, *args):
+            if name == "ng_lm_index":
+                x, act, n, length, k0, table, cap_q, slots, rep, base, fid, counters = args
+                args = (x, act, n, length, k0, table, LG.u64(1), LG.u64(room), rep, base, fid, counters)
+                super().__call__(name, *args)
+                at = act[:n].long()
+                assert bool((counters[:, 1] != 0).any()) and bool((fid[at][length[at] >= k0.value] == -1).any())
+                return 0
+            return super().__call__(name, *args)
+
+    monkeypatch.setattr(LG, "_WIDE", set())
+    monkeypatch.setattr(LG, "_count_wide", wide)
+    for room in (2, 8):  # the last slot stays empty
+        again.clear()
+        got = longest_match(tok, xt, av, 64, elib=Small())
+        assert again == [["lists"]] and not LG._WIDE
+        for g, w in zip(got[:3], want[:3]):
+            assert torch.equal(g, w)
 
 
 def test_ladder_interface(corpus, tmp_path):
