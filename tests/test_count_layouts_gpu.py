@@ -2,6 +2,8 @@
 they go below it, and at the most it takes, against the oracle: with and without records in runs, top 1 and top 8, one
 query position and many."""
 
+import math
+
 import numpy as np
 import pytest
 
@@ -44,8 +46,16 @@ def test_partition_layouts(corpus, target, pbits, topk, queries, runs, monkeypat
             assert np.array_equal(out[2, li].view(np.uint32), o["cnt"]), f"cnt k={k}"
             assert np.array_equal(cb.top_tok[li].cpu().numpy().view(np.uint16), o["top_tok"][:, :topk]), f"top k={k}"
             assert np.array_equal(cb.top_cnt[li].cpu().numpy().view(np.uint32), o["top_cnt"][:, :topk]), f"top k={k}"
-    if queries > 1:
-        assert cb.info[2]["pbits"] >= min(pbits, P.pbits32_max(cb.info[2]["ids"])) and not cb.engine.wide
-    if target == 1 << 30:
-        assert all(cb.info[k]["pbits"] == P.first_digit(P.w_bits(cb.info[k]["ids"])[1]) or k not in cb.engine.min_pbits
-                   for k in LEVELS)
+    # the second build's partitions, sized from the first one's events and pairs: the first pass's digit itself where they
+    # fit it, else at least PART_MIN_BITS
+    taken = set()
+    for k in LEVELS:
+        idb, W = P.w_bits(cb.info[k]["ids"])
+        d1, by_range = P.first_digit(W), runs and P.runs_fit(cb.info[k]["ids"], topk)
+        used = cb.info[k]["ids"] / (1 << idb) if by_range else 1.0
+        want = math.ceil(math.log2(max(1.0, cb.info[k]["pairs"] / target / used)))
+        want = max(want, P.PART_MIN_BITS) if want > d1 else d1
+        assert cb.info[k]["pbits"] == min(want, P.pbits32_max(cb.info[k]["ids"])), f"k={k}"
+        taken.add(cb.info[k]["pbits"])
+    assert not cb.engine.wide and not cb.engine.min_pbits  # none was counted again with more
+    assert taken == {8} if target == 1 << 30 else queries == 1 or max(taken) >= pbits
