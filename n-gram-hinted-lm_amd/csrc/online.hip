@@ -960,23 +960,28 @@ __device__ __forceinline__ i64 opart(const i64* __restrict__ bounds, i64 np, i64
 }
 
 // tau[p] = min over the spans (lo, hi, step) [m, 3] that hold p of their step; item i of the spans' lengths laid end
-// to end (offs: their exclusive sums, offs[m] = total), OTAU_ITEMS a thread, so that one long span takes many blocks.
+// to end (offs: their exclusive sums, offs[m] = total), OTAU_ITEMS a thread, so that one long span takes many blocks, and
+// OTAU_BLOCKS blocks at most, which then go round: spans may overlap, so their lengths are not bounded by the stream's, and
+// a launch of 2^32 threads or more runs only some of them.
+#define OTAU_BLOCKS (1 << 20)
 __global__ void __launch_bounds__(256) online_tau_k(const i64* __restrict__ spans, const i64* __restrict__ offs, i64 m,
                                                     u32* tau) {
     const i64 total = offs[m];
-    i64 i = (blockIdx.x * (i64)blockDim.x + threadIdx.x) * OTAU_ITEMS;
-    if (i >= total) return;
-    const i64 end = i + OTAU_ITEMS < total ? i + OTAU_ITEMS : total;
-    i64 a = 0, b = m;  // offs[a] <= i < offs[b]: the last such a is the span
-    while (b - a > 1) {
-        const i64 c = (a + b) >> 1;
-        if (offs[c] <= i) a = c;
-        else b = c;
-    }
-    for (; i < end; ++a) {
-        const i64 lo = spans[3 * a], stop = offs[a + 1] < end ? offs[a + 1] : end;
-        const u32 step = (u32)spans[3 * a + 2];
-        for (; i < stop; ++i) atomicMin(&tau[lo + (i - offs[a])], step);
+    for (i64 i0 = (blockIdx.x * (i64)blockDim.x + threadIdx.x) * OTAU_ITEMS; i0 < total;
+         i0 += (i64)gridDim.x * blockDim.x * OTAU_ITEMS) {
+        i64 i = i0;
+        const i64 end = i + OTAU_ITEMS < total ? i + OTAU_ITEMS : total;
+        i64 a = 0, b = m;  // offs[a] <= i < offs[b]: the last such a is the span
+        while (b - a > 1) {
+            const i64 c = (a + b) >> 1;
+            if (offs[c] <= i) a = c;
+            else b = c;
+        }
+        for (; i < end; ++a) {
+            const i64 lo = spans[3 * a], stop = offs[a + 1] < end ? offs[a + 1] : end;
+            const u32 step = (u32)spans[3 * a + 2];
+            for (; i < stop; ++i) atomicMin(&tau[lo + (i - offs[a])], step);
+        }
     }
 }
 
@@ -1041,8 +1046,8 @@ extern "C" int ng_online_tau(const i64* spans, const i64* offs, i64 m, i64 total
     hipStream_t st = (hipStream_t)stream;
     int e = prim::fill_u32(tau_in, 0xFFFFFFFFu, n, st);
     if (e) return e;
-    const i64 items = (total + OTAU_ITEMS - 1) / OTAU_ITEMS;
-    if (total) online_tau_k<<<grid_for(items, 256), 256, 0, st>>>(spans, offs, m, tau_in);
+    const i64 blocks = (total + OTAU_ITEMS * 256 - 1) / (OTAU_ITEMS * 256);
+    if (total) online_tau_k<<<(int)(blocks < OTAU_BLOCKS ? blocks : OTAU_BLOCKS), 256, 0, st>>>(spans, offs, m, tau_in);
     if ((e = (int)hipMemcpyAsync(tau, tau_in, (size_t)n * 4, hipMemcpyDeviceToDevice, st))) return e;
     if (m) online_targets_k<<<grid_for(m, 256), 256, 0, st>>>(spans, m, bounds, np, n, tau);
     return (int)hipGetLastError();

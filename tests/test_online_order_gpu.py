@@ -76,3 +76,18 @@ def test_bounds_of_steps_close_together_and_apart(gpu, m, top, monkeypatch):
         for s in (0, 1, top // 2, top, *steps[:50].tolist()):
             assert b1.before(int(s)) == b2.before(int(s)), s
     assert rows._most([b for _, b in got[0]]) == rows._most([b for _, b in list(got.values())[0]])
+
+
+@pytest.mark.parametrize("times", [3, 70_000])
+def test_spans_that_cover_the_stream_many_times(gpu, times):
+    """Spans overlap freely, so their lengths add up to far more than the stream: at 70,000 times 2^20 positions to more
+    than a launch has threads for (16 positions each)."""
+    n = 1 << 20
+    rng = np.random.default_rng(times)
+    lo = rng.integers(0, 50, times)
+    steps = rng.permutation(np.arange(5, 5 + times))
+    rows = OnlineRows(np.zeros(n, np.uint16), [0, n], np.stack([lo, np.full(times, n), steps], 1))
+    want = np.full(n, steps.min(), np.int64)
+    for g in range(50):
+        want[g] = steps[lo <= g].min() if (lo <= g).any() else NONE
+    assert np.array_equal(rows.tau_in.cpu().numpy().view(np.uint32), want)
