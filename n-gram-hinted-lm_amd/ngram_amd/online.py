@@ -158,7 +158,9 @@ class OnlineRows:
                  self.tau_in)
         self.max_step = int(sp[:, 2].max()) if len(sp) else -1
         self.max_steps = len(sp)  # at most this many steps are in use
-        self._trained = None  # how many positions have a step, once asked for
+        # at most how many positions have a step: of spans in order without overlap, theirs and each one's last target; else
+        # counted once it is asked for (about 70 us)
+        self._trained = min(n, int(offs[-1]) + len(sp)) if (sp[1:, 0] >= sp[:-1, 1]).all() else None
         seg = torch.empty(n, dtype=torch.int64, device=dev)
         self.has_next = torch.empty(n, dtype=torch.uint8, device=dev)
         self.lib("ng_online_layout", self.tok, n, self.bounds_dev, np_, seg, self.has_next)

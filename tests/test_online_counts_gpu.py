@@ -53,7 +53,8 @@ def test_calls_at_the_edge_of_what_is_taken(gpu):
 
 @pytest.mark.parametrize("trained", [0, 1, 2, 300, 4800])
 @pytest.mark.parametrize("spread", [1, 3_000_000])
-def test_a_stream_of_which_few_positions_are_trained(gpu, trained, spread, monkeypatch):
+@pytest.mark.parametrize("in_order", [True, False])
+def test_a_stream_of_which_few_positions_are_trained(gpu, trained, spread, in_order, monkeypatch):
     """Picking the trained positions out before they are sorted gives the state and the count rows that sorting the whole
     stream gives, and keeps lists only as long as they are."""
     n, m = 20_000, max(1, trained // 40)
@@ -61,12 +62,14 @@ def test_a_stream_of_which_few_positions_are_trained(gpu, trained, spread, monke
     tok = rng.integers(0, 6, n).astype(np.uint16)
     tok[rng.random(n) < 0.01] = 50256
     at = rng.choice(n // 50 - 1, m, replace=False) * 50
+    if in_order:
+        at = np.sort(at)
     size = np.full(m, 40) if trained >= 40 else np.full(m, trained)
     spans = np.stack([at, at + size, rng.integers(0, 7, m) * spread], 1)
     got = {}
     for few in (1, 1 << 40):
         monkeypatch.setattr(online, "FEW_MIN", few)
-        rows = OnlineRows(tok, [0, n // 3, n], spans)
+        rows = OnlineRows(tok, [0, n // 3, n], spans if few == 1 else spans[::-1])  # in order (or not), and the other way
         rows.prepare([1, 3], [1, 3], 4, [1, 3, 9])
         lists = [rows.state["q_pos"]] + [lv["occ"] for lv in rows.state["levels"].values()]
         out = [np.zeros((n, 3), t) for t in (np.uint32, np.uint16, np.uint32)]
